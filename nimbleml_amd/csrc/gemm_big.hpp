@@ -52,6 +52,17 @@ __device__ __forceinline__ int xcd_tile(int b, int tiles) {
   return x * per + (x < rem ? x : rem) + (b >> 3);
 }
 
+// Output position of tile t: GM m-bands per group, m fastest inside a group.
+template <int GM>
+__device__ __forceinline__ void tile_at(int t, int tiles_n, int tiles, int TM, int TN, int* m0, int* n0) {
+  const int tiles_m = tiles / tiles_n;
+  const int group = t / (GM * tiles_n), first = group * GM;
+  const int gm = tiles_m - first < GM ? tiles_m - first : GM;
+  const int in = t - group * GM * tiles_n;
+  *m0 = (first + in % gm) * TM;
+  *n0 = (in / gm) * TN;
+}
+
 // s_waitcnt lgkmcnt(IA + JB) (the step just issued may stay outstanding) or lgkmcnt(0),
 // with the fragments passed through so that no use is moved above the wait.
 template <int IA, int JB>

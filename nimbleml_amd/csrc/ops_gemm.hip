@@ -4,10 +4,10 @@
 // GEMM operands are K-major (the natural MFMA operand layout) and a decode GEMV
 // streams each output's weights as one contiguous row.
 //
-//  * gemm_f16 / gemm_f32: 128×128 block tile, 4 waves as 2×2, each wave 64×64 as
-//    2×2 MFMA 32×32 tiles (fp16: v_mfma_f32_32x32x16_f16, K=64 per LDS stage;
-//    fp32: v_mfma_f32_32x32x2f32, K=32 per stage). Next stage prefetched into
-//    registers while the current one is multiplied.
+//  * gemm_f16: 128×128 block tile, 4 waves as 2×2, each wave 64×64 as 2×2 MFMA tiles
+//    (v_mfma_f32_32x32x16_f16, K=64 per LDS stage). Next stage prefetched into registers
+//    while the current one is multiplied.
+//  * gemm_f32: every float32 value split into three bf16 parts (gemm_split.hpp).
 //  * gemv: M ≤ 8 activation rows (decode). One wave per output row (or four),
 //    16-byte loads along K, fp32 accumulation, wave-reduced.
 //  * skinny_f16: 8 < M ≤ 64 rows (batched decode), MFMA 16×16×32 with optional split-K
@@ -15,7 +15,7 @@
 #include <cstdlib>
 #include <mutex>
 
-#include "gemm_big.hpp"
+#include "gemm_split.hpp"
 #include "kernels.hpp"
 
 namespace nml {
@@ -707,12 +707,8 @@ __global__ __launch_bounds__(kHT, TM == 256 ? 1 : 4) void gemm_f16_big_kernel(Li
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
   const int wm = wave >> 2, wn = wave & 3;  // 2 × 4 waves of TM/2 × TN/4
   // XCD-aware tile order, GM m-bands per group
-  const int t = big::xcd_tile(blockIdx.x, tiles);
-  const int tiles_m = tiles / tiles_n;
-  const int group = t / (GM * tiles_n), first = group * GM;
-  const int gm = tiles_m - first < GM ? tiles_m - first : GM;
-  const int in = t - group * GM * tiles_n;
-  const int m0 = (first + in % gm) * TM, n0 = (in / gm) * TN;
+  int m0, n0;
+  big::tile_at<GM>(big::xcd_tile(blockIdx.x, tiles), tiles_n, tiles, TM, TN, &m0, &n0);
 
   floatx16 acc[IA][JB];
 #pragma unroll
@@ -799,88 +795,40 @@ bool big_gemm_applies(const LinearArgs& a) {
   return a.M >= 256 && !(std::getenv("NIMBLEML_BIG_GEMM") && std::getenv("NIMBLEML_BIG_GEMM")[0] == 'w');
 }
 
-// ---------------------------------------------------------------- fp32 MFMA GEMM
-constexpr int kBK32 = 32, kPad32 = 4;
+// ------------------------------------------------ fp32 GEMM on the bf16 matrix cores
+// x3::tile (gemm_split.hpp) with the projection epilogues; tiles ordered XCD by XCD, 4
+// m-bands at a time, as the fp16 GEMM's.
+template <int EPI, int TM, int TN, int WM, int WN, int WK>
+__global__ __launch_bounds__(64 * WM * WN * WK, 2) void gemm_f32_kernel(LinearArgs a, int tiles_n, int tiles) {
+  extern __shared__ __attribute__((aligned(1024))) char lds_raw[];
+  int m0, n0;
+  big::tile_at<4>(big::xcd_tile(blockIdx.x, tiles), tiles_n, tiles, TM, TN, &m0, &n0);
+  x3::tile<TM, TN, WM, WN, WK, true, true>(
+      x3::Operand{static_cast<const float*>(a.x), a.lda}, x3::Operand{static_cast<const float*>(a.w), a.K},
+      a.M, a.N, m0, n0, 0, a.K, lds_raw,
+      [&](int m, int n, float v) { epilogue<float, EPI>(a, m, n, v); });
+}
+
+template <int EPI, int TM, int TN, int WM, int WN, int WK>
+int gemm_f32_launch_tile(const LinearArgs& a, hipStream_t st) {
+  typedef x3::Shape<TM, TN, WM, WN, WK> Sh;
+  static bool attr = false;
+  if (!attr) {
+    NML_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_kernel<EPI, TM, TN, WM, WN, WK>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(Sh::Lds)));
+    attr = true;
+  }
+  const int tiles_n = (a.N + TN - 1) / TN, tiles = tiles_n * ((a.M + TM - 1) / TM);
+  gemm_f32_kernel<EPI, TM, TN, WM, WN, WK><<<tiles, Sh::Threads, Sh::Lds, st>>>(a, tiles_n, tiles);
+  NML_LAUNCHED();
+  return 0;
+}
 
 template <int EPI>
-__global__ __launch_bounds__(256) void gemm_f32_kernel(LinearArgs a) {
-  __shared__ float As[kBM][kBK32 + kPad32];
-  __shared__ float Bs[kBN][kBK32 + kPad32];
-  const float* __restrict__ X = static_cast<const float*>(a.x);
-  const float* __restrict__ W = static_cast<const float*>(a.w);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int m0 = blockIdx.y * kBM, n0 = blockIdx.x * kBN;
-  const int M = a.M, N = a.N, K = a.K;
-  const long long lda = a.lda;
-
-  floatx16 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-  floatx4 ra[4], rb[4];
-  const floatx4 zero4 = {0.f, 0.f, 0.f, 0.f};
-  auto gload = [&](int k0) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int c = tid + 256 * i;
-      const int row = c >> 3, kc = (c & 7) * 4;
-      const int gk = k0 + kc;
-      const int gm = m0 + row, gn = n0 + row;
-      ra[i] = (gm < M && gk < K) ? *reinterpret_cast<const floatx4*>(X + gm * lda + gk) : zero4;
-      rb[i] = (gn < N && gk < K)
-                  ? *reinterpret_cast<const floatx4*>(W + static_cast<long long>(gn) * K + gk)
-                  : zero4;
-    }
-  };
-  auto sstore = [&]() {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int c = tid + 256 * i;
-      const int row = c >> 3, kc = (c & 7) * 4;
-      *reinterpret_cast<floatx4*>(&As[row][kc]) = ra[i];
-      *reinterpret_cast<floatx4*>(&Bs[row][kc]) = rb[i];
-    }
-  };
-
-  gload(0);
-  sstore();
-  __syncthreads();
-  for (int k0 = 0; k0 < K; k0 += kBK32) {
-    const bool more = k0 + kBK32 < K;
-    if (more) gload(k0 + kBK32);
-#pragma unroll
-    for (int kk = 0; kk < kBK32; kk += 2) {
-      float fa[2], fb[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) fa[i] = As[wm * 64 + i * 32 + (lane & 31)][kk + (lane >> 5)];
-#pragma unroll
-      for (int j = 0; j < 2; ++j) fb[j] = Bs[wn * 64 + j * 32 + (lane & 31)][kk + (lane >> 5)];
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i], fb[j], acc[i][j], 0, 0, 0);
-    }
-    __syncthreads();
-    if (more) sstore();
-    __syncthreads();
-  }
-
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int m = m0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        const int n = n0 + wn * 64 + j * 32 + (lane & 31);
-        if (m < M && n < N) epilogue<float, EPI>(a, m, n, acc[i][j][r]);
-      }
+int gemm_f32_launch(const LinearArgs& a, hipStream_t st) {
+  const long long big = ((a.M + 127LL) / 128) * ((a.N + 127LL) / 128);
+  if (big >= x3::kLargeTiles) return gemm_f32_launch_tile<EPI, 128, 128, 2, 2, 2>(a, st);
+  return gemm_f32_launch_tile<EPI, 64, 64, 1, 2, 2>(a, st);
 }
 
 // --------------------------------------------------------------------- GEMV
@@ -1428,12 +1376,12 @@ int linear_typed(const LinearArgs& a, hipStream_t st) {
   }
   if constexpr (sizeof(T) == 2) {
     if (big_gemm_applies(a)) return gemm_big_launch<EPI>(a, st);
+  } else {
+    return gemm_f32_launch<EPI>(a, st);
   }
   dim3 grid((a.N + kBN - 1) / kBN, (a.M + kBM - 1) / kBM);
   if constexpr (sizeof(T) == 2)
     gemm_f16_kernel<EPI><<<grid, 256, 0, st>>>(a);
-  else
-    gemm_f32_kernel<EPI><<<grid, 256, 0, st>>>(a);
   NML_LAUNCHED();
   return 0;
 }

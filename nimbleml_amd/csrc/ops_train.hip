@@ -7,9 +7,11 @@
 // gradients accumulate in fp32, and the fp16 branches keep the reference's fp16 rounding
 // points where the reference writes them op by op (RMSNorm, GELU, cross-entropy, RoPE).
 //
-//  * gemm_bwd_kernel: 128 × 128 tile, 4 waves of 64 × 64, MFMA 32×32×2 fp32; either
-//    operand read k-contiguous (rows of a row-major matrix) or m/n-contiguous (columns),
-//    staged through LDS as [k][row] so every MFMA fragment read is a contiguous row.
+//  * float32 products: x3::tile (gemm_split.hpp), every value split into three bf16 parts;
+//    either operand k-contiguous (rows of a row-major matrix) or m/n-contiguous (columns).
+//  * gemm_bwd_kernel (fp16 operands whose extents are no multiple of 8): 128 × 128 tile, 4
+//    waves of 64 × 64, MFMA 32×32×2 fp32, staged through LDS as [k][row] so every MFMA
+//    fragment read is a contiguous row.
 //  * attention backward: per (sequence, head), one kernel owns a tile of keys and
 //    walks the queries after it (dK, dV), another owns a tile of queries and walks the
 //    keys before it (dQ); both recompute P = exp(q·k/√dk − lse) from the forward's
@@ -18,7 +20,7 @@
 //    and a second pass in a fixed order: the result does not depend on scheduling.
 #include <cstdlib>
 
-#include "gemm_big.hpp"
+#include "gemm_split.hpp"
 #include "kernels.hpp"
 
 namespace nml {
@@ -622,6 +624,91 @@ int gemm_bwd_big(const GemmBwdArgs& g0, bool a_kc, bool b_kc, int out, hipStream
   p.ldc = g.N;
   NML_TRY((big_bwd_out<128, 128>(p, kGBPart, splits, kchunk, M * N, st)));
   splitk_reduce_kernel<half_t><<<static_cast<int>((M * N + 255) / 256), 256, 0, st>>>(
+      g_split.p, splits, g.M, g.N, static_cast<float*>(g.c), g.ldc);
+  NML_LAUNCHED();
+  return 0;
+}
+
+// float32 products on x3::tile (gemm_split.hpp): block b → (tile, split) through the
+// XCD-aware order, output modes as gemm_bwd_kernel.
+template <int TM, int TN, int WM, int WN, int WK, bool A_KC, bool B_KC, int OUT>
+__global__ __launch_bounds__(64 * WM * WN * WK, 2) void gemm_bwd_f32_kernel(GemmBwdArgs g, int tiles_n, int tiles,
+                                                                          int splits, int kchunk, long long zstride) {
+  extern __shared__ __attribute__((aligned(1024))) char lds_raw[];
+  const int u = big::xcd_tile(blockIdx.x, tiles * splits);
+  const int z = u % splits;
+  int m0, n0;
+  big::tile_at<4>(u / splits, tiles_n, tiles, TM, TN, &m0, &n0);
+  const int kbeg = z * kchunk, kend = min(g.K, kbeg + kchunk);
+  float* c = static_cast<float*>(g.c) + (OUT == kGBPart ? z * zstride : 0);
+  x3::tile<TM, TN, WM, WN, WK, A_KC, B_KC>(
+      x3::Operand{static_cast<const float*>(g.a), g.lda}, x3::Operand{static_cast<const float*>(g.b), g.ldb},
+      g.M, g.N, m0, n0, kbeg, kend, lds_raw, [&](int m, int n, float v) {
+        const long long ci = static_cast<long long>(m) * g.ldc + n;
+        if constexpr (OUT == GB_ADD) v += c[ci];
+        if constexpr (OUT == GB_GELU)
+          v *= gelu_grad(static_cast<const float*>(g.aux)[static_cast<long long>(m) * g.ldaux + n]);
+        c[ci] = v;
+      });
+}
+
+template <int TM, int TN, int WM, int WN, int WK, bool A_KC, bool B_KC, int OUT>
+int gemm_bwd_f32_launch(const GemmBwdArgs& g, int splits, int kchunk, hipStream_t st) {
+  typedef x3::Shape<TM, TN, WM, WN, WK> Sh;
+  static bool attr = false;
+  if (!attr) {
+    NML_HIP(hipFuncSetAttribute(
+        reinterpret_cast<const void*>(&gemm_bwd_f32_kernel<TM, TN, WM, WN, WK, A_KC, B_KC, OUT>),
+        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(Sh::Lds)));
+    attr = true;
+  }
+  const int tiles_n = (g.N + TN - 1) / TN, tiles = tiles_n * ((g.M + TM - 1) / TM);
+  gemm_bwd_f32_kernel<TM, TN, WM, WN, WK, A_KC, B_KC, OUT><<<tiles * splits, Sh::Threads, Sh::Lds, st>>>(
+      g, tiles_n, tiles, splits, kchunk, static_cast<long long>(g.M) * g.N);
+  NML_LAUNCHED();
+  return 0;
+}
+
+template <bool A_KC, bool B_KC, int OUT>
+int gemm_bwd_f32_tile(const GemmBwdArgs& g, bool large, int splits, int kchunk, hipStream_t st) {
+  if (large) return gemm_bwd_f32_launch<128, 128, 2, 2, 2, A_KC, B_KC, OUT>(g, splits, kchunk, st);
+  return gemm_bwd_f32_launch<64, 64, 1, 2, 2, A_KC, B_KC, OUT>(g, splits, kchunk, st);
+}
+
+// K split (accumulating outputs, the weight gradients, whose K is the row count) until the
+// grid holds a workgroup of 128 × 128 per CU, each slice ≥ 256 long; partials summed in
+// a fixed order.
+template <bool A_KC, bool B_KC>
+int gemm_bwd_f32(const GemmBwdArgs& g, int out, hipStream_t st) {
+  const long long big = ((g.M + 127LL) / 128) * ((g.N + 127LL) / 128);
+  int splits = 1;
+  if (out == GB_ADD)
+    while (splits < 16 && big * splits < 256 && g.K / (2 * splits) >= 256) splits *= 2;
+  const bool large = big * splits >= x3::kLargeTiles;
+  const int kchunk = ((g.K + splits - 1) / splits + x3::kK - 1) / x3::kK * x3::kK;
+  splits = (g.K + kchunk - 1) / kchunk;  // no empty slice
+  if (splits == 1) {
+    switch (out) {
+      case GB_SET: return gemm_bwd_f32_tile<A_KC, B_KC, GB_SET>(g, large, 1, kchunk, st);
+      case GB_ADD: return gemm_bwd_f32_tile<A_KC, B_KC, GB_ADD>(g, large, 1, kchunk, st);
+      case GB_GELU: return gemm_bwd_f32_tile<A_KC, B_KC, GB_GELU>(g, large, 1, kchunk, st);
+      default: set_error("gemm_bwd: unknown output mode %d", out); return -1;
+    }
+  }
+  const size_t need = static_cast<size_t>(splits) * g.M * g.N;
+  if (need > g_split.floats) {
+    NML_HIP(hipStreamSynchronize(st));
+    if (g_split.p) NML_HIP(hipFree(g_split.p));
+    g_split = SplitWs{};
+    NML_HIP(hipMalloc(&g_split.p, need * sizeof(float)));
+    g_split.floats = need;
+  }
+  GemmBwdArgs p = g;
+  p.c = g_split.p;
+  p.ldc = g.N;
+  NML_TRY((gemm_bwd_f32_tile<A_KC, B_KC, kGBPart>(p, large, splits, kchunk, st)));
+  const long long mn = static_cast<long long>(g.M) * g.N;
+  splitk_reduce_kernel<float><<<static_cast<int>((mn + 255) / 256), 256, 0, st>>>(
       g_split.p, splits, g.M, g.N, static_cast<float*>(g.c), g.ldc);
   NML_LAUNCHED();
   return 0;
@@ -2165,8 +2252,8 @@ int launch_gemm_bwd(int dt, const GemmBwdArgs& g, bool a_kc, bool b_kc, int out,
       return b_kc ? gemm_bwd_out<true, true, half_t>(g, out, st, m16) : gemm_bwd_out<true, false, half_t>(g, out, st, m16);
     return b_kc ? gemm_bwd_out<false, true, half_t>(g, out, st, m16) : gemm_bwd_out<false, false, half_t>(g, out, st, m16);
   }
-  if (a_kc) return b_kc ? gemm_bwd_out<true, true, float>(g, out, st) : gemm_bwd_out<true, false, float>(g, out, st);
-  return b_kc ? gemm_bwd_out<false, true, float>(g, out, st) : gemm_bwd_out<false, false, float>(g, out, st);
+  if (a_kc) return b_kc ? gemm_bwd_f32<true, true>(g, out, st) : gemm_bwd_f32<true, false>(g, out, st);
+  return b_kc ? gemm_bwd_f32<false, true>(g, out, st) : gemm_bwd_f32<false, false>(g, out, st);
 }
 
 int launch_convert(int src_dt, const void* src, int dst_dt, void* dst, size_t n, hipStream_t st) {

@@ -1,0 +1,87 @@
+"""float32 products on the bf16 matrix cores (csrc/gemm_split.hpp): the forward projection and
+both backward products against float64, at the edges of the 64 and 128 wide tiles and of the
+32-wide k stages; outputs that need the float32 slow path; and the sums' freedom from bias."""
+import numpy as np
+import pytest
+
+from nimbleml_amd import _native as N
+from nimbleml_amd import kernels as K
+
+pytestmark = pytest.mark.gpu
+
+
+def bound(x, y, k):
+    """Σ|x||y| times the roundings of a k-term sum taken 16 terms at a time (two partial sums
+    and their total on top), plus the dropped products' 2^-25."""
+    return (np.abs(x).astype(np.float64) @ np.abs(y).astype(np.float64)) * ((k / 16 + 4) * 2.0**-24)
+
+
+# rows: the first past the skinny path, tile edges and one past them, enough 128 × 128 tiles
+# for the large-tile kernel; k: below, at and past a stage, odd multiples of 4, past the
+# 512-term accumulator
+@pytest.mark.parametrize("rows,n,k", [(65, 64, 4), (127, 65, 28), (128, 192, 32), (129, 129, 36),
+                                      (200, 4096, 68), (70, 31, 1060), (1665, 1793, 100),
+                                      (1536, 2048, 544)])
+def test_linear_f32_against_float64(rows, n, k):
+    r = np.random.RandomState(rows + n + k)
+    x, w = r.randn(rows, k).astype(np.float32), r.randn(k, n).astype(np.float32)
+    got = K.linear(x, w).numpy()
+    want = x.astype(np.float64) @ w.astype(np.float64)
+    assert (np.abs(got - want) <= bound(x, w, k)).all()
+
+
+def backward(dy, x, w):
+    """(dx, dw) of y = x·w with w (in, out)."""
+    rows, out = dy.shape
+    d = [N.DeviceArray.from_host(a) for a in (dy, x, np.ascontiguousarray(w.T))]
+    dx = N.DeviceArray(x.shape, np.float32)
+    dw = N.DeviceArray.from_host(np.zeros((out, x.shape[1]), np.float32))
+    N.check(N.lib.nml_linear_backward_device(d[0].ptr, d[1].ptr, d[2].ptr, dx.ptr, dw.ptr, None,
+                                             rows, x.shape[1], out, None, 0))
+    return dx.numpy(), dw.numpy().T
+
+
+@pytest.mark.parametrize("rows,n_in,n_out", [(1, 4, 8), (33, 64, 68), (129, 132, 60),
+                                             (1027, 256, 192), (2100, 1668, 1540)])
+def test_backward_f32_against_float64(rows, n_in, n_out):
+    r = np.random.RandomState(rows)
+    dy, x = r.randn(rows, n_out).astype(np.float32), r.randn(rows, n_in).astype(np.float32)
+    w = r.randn(n_in, n_out).astype(np.float32)
+    dx, dw = backward(dy, x, w)
+    d64 = dy.astype(np.float64)
+    assert (np.abs(dx - d64 @ w.T) <= bound(dy, w.T, n_out)).all()
+    assert (np.abs(dw - x.T.astype(np.float64) @ d64) <= bound(x.T, dy, rows)).all()
+
+
+@pytest.mark.parametrize("rows,n", [(96, 96), (1665, 1793)])
+def test_infinite_nan_and_largest_values(rows, n):
+    """Outputs as float32 multiply-adds give them where a value is infinite, NaN, or rounds
+    up to infinity in bf16; every other output is untouched."""
+    r = np.random.RandomState(7)
+    k = 72
+    x, w = r.randn(rows, k).astype(np.float32), r.randn(k, n).astype(np.float32)
+    big = np.finfo(np.float32).max
+    x[3, 5], x[8, 70], x[rows - 1, 0] = np.inf, np.nan, -np.inf
+    x[20], x[20, 11] = 0.0, big      # one huge term: finite where its weight is below one
+    w[11, 2] = 0.25
+    got = K.linear(x, w).numpy()
+    with np.errstate(all="ignore"):
+        want = x.astype(np.float64) @ w.astype(np.float64)
+        want = np.where(np.abs(want) > big, np.sign(want) * np.inf, want)
+    same = np.isnan(want) == np.isnan(got)
+    assert same.all() and (np.isinf(want) == np.isinf(got)).all()
+    assert (got[np.isinf(want)] == want[np.isinf(want)]).all()
+    assert got[20, 2] == np.float32(big) * np.float32(0.25)
+    plain = np.setdiff1d(np.arange(rows), [3, 8, 20, rows - 1])
+    assert (np.abs(got[plain] - want[plain]) <= bound(x[plain], w, k)).all()
+
+
+def test_sums_have_no_common_bias():
+    """A column sum over many rows must not gather one-sided rounding: each output's error
+    is independent, so the mean over 4096 rows falls like 1/sqrt(4096). Four standard errors
+    of the mean, over the worst of 64 columns."""
+    r = np.random.RandomState(3)
+    rows, k, n = 4096, 1024, 64
+    x, w = r.rand(rows, k).astype(np.float32), r.randn(k, n).astype(np.float32)
+    err = K.linear(x, w).numpy() - x.astype(np.float64) @ w.astype(np.float64)
+    assert (np.abs(err.mean(0)) <= 6 * err.std(0) / np.sqrt(rows)).all()
