@@ -6,13 +6,13 @@
 // fp16 divisor); the softmax itself runs online in fp32 (flash form), so no
 // (S, S) score matrix exists.
 //
-//  * prefill, fp16 head dim 64/128: MFMA flash attention, 128 queries per workgroup,
-//    64-key K/V tiles in LDS — attn_prefill_pipe_kernel (fp32 scores, software-pipelined
-//    over the tiles) where no statistics are kept, attn_prefill_mfma_kernel (fp16-rounded
-//    scores, statistics for the backward) otherwise;
-//    fp32 head dim 64/128: attn_prefill_f32_mfma; head dims 8/16/32 (and the non-causal
-//    masked form): attn_prefill_kernel, one wave per 64 queries, scalar; any other head
-//    dim ≤ 256: attn_prefill_quad_kernel, four lanes per query.
+//  * prefill, head dims up to 128 in 16-byte pieces: MFMA flash attention, 128 queries per
+//    workgroup, 64-key K/V tiles in LDS, causal, full or masked — fp16
+//    attn_prefill_pipe_kernel (fp32 scores, software-pipelined over the tiles) where no
+//    statistics are kept, attn_prefill_mfma_kernel (fp16-rounded scores, statistics for the
+//    backward; causal, head dim 64/128); fp32 attn_prefill_f32_mfma;
+//    the rest: head dims 8/16/32/64/128 attn_prefill_kernel, one wave per 64 queries,
+//    scalar; any other head dim ≤ 256 attn_prefill_quad_kernel, four lanes per query.
 //  * decode, head dim 32/64/128/256: attn_decode_group_kernel — split-K in one launch:
 //    each workgroup scores a group of 64-key chunks of one (sequence, head) and publishes
 //    its (max, Σp, Σp·v) as flagged slots; the last workgroup of the (sequence, head)
@@ -785,7 +785,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_kernel(AttnArgs a) {
   }
 }
 
-// Causal flash attention on the matrix cores with fp32 scores (prefill calls that keep
+// Flash attention on the matrix cores with fp32 scores (prefill calls that keep
 // no softmax statistics), software-pipelined over the 64-key tiles. The layout per wave
 // is attn_prefill_mfma_kernel's (32 queries, Sᵀ = K·Qᵀ and Oᵀ += Vᵀ·Pᵀ on
 // v_mfma_f32_32x32x16_f16, each lane owning one query's softmax state and output
@@ -802,13 +802,31 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_kernel(AttnArgs a) {
 // Rows past the last key are read clamped to it (in bounds and finite; the causal
 // mask removes them), so a tile needs no bounds tests. Waves whose queries all lie
 // past the sequence skip the arithmetic but join the barriers.
-template <int DK>
+//
+// MODE: causal; full (every key); or full with an additive (S, S) mask. PAD: the head dim
+// a.dk (a multiple of 8) is below DK: dims past it read as zero and are not stored. EXACT: the
+// probabilities enter P·V as two fp16 parts (22 bits) and two products, for the calls that
+// took float32 probabilities from the scalar kernels before (every one but causal head dims
+// 64 and 128); their scores stay float32 accumulators, except that a masked score is rounded
+// as the reference's fp16 ops round it, rnd(rnd(rnd(q·k) / scale) + mask): a mask of the
+// type's lowest value must absorb the score. A tile whose keys are all −∞ for a query leaves
+// its reference point at −∞ and adds nothing; a query with no other key gives NaN, as a
+// softmax over nothing does.
+// 4 × 16 heads × 1024 keys of 64 dims, every key: the scalar kernel's 826 µs fell to 42 (410
+// TFLOP/s of the algorithm's two products), masked to 77; 4 × 8 heads of 128: 45 and 86. The
+// masked form is held by the mask's loads, waited for in every tile, and by its four
+// rounding operations a score.
+enum AttnMode : int { kCausal = 0, kFull = 1, kMasked = 2 };
+
+template <int DK, int MODE, bool PAD, bool EXACT>
 __global__ __launch_bounds__(256, 2) void attn_prefill_pipe_kernel(AttnArgs a) {
 #pragma clang fp contract(off)
   constexpr int KS = DK / 16;  // 16-dim steps of q·k
   constexpr int OT = DK / 32;  // 32-dim tiles of the output
-  constexpr int CH = kFK * DK / 8 / 256;  // 16-byte pieces of a tile's K (and of V) per thread
+  constexpr int CH = kFK * DK / 8 / 256;  // 16-byte pieces of a tile's K per thread
   constexpr int VG = DK / 8;              // 8-dim groups of a key
+  constexpr int VI = (VG + 7) / 8;        // V: 8-dim groups per thread, each for two keys
+  const int dk = PAD ? a.dk : DK;         // row length of q, k and v
   __shared__ half_t Ks[2][kFK][DK + 8];
   __shared__ half_t Vt[2][DK][kFK + 4];  // rows 34 dwords apart, as in attn_prefill_mfma_kernel
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -827,10 +845,11 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pipe_kernel(AttnArgs a) {
   const int base = a.pos_base ? a.pos_base[b] : 0;
   const half_t* __restrict__ Kg = static_cast<const half_t*>(a.k) + b * a.kv_stride_b + h * a.kv_stride_h;
   const half_t* __restrict__ Vg = static_cast<const half_t*>(a.v) + b * a.kv_stride_b + h * a.kv_stride_h;
-  const half_t* __restrict__ Qg = static_cast<const half_t*>(a.q) + static_cast<size_t>(bh) * a.S * DK;
+  const half_t* __restrict__ Qg = static_cast<const half_t*>(a.q) + static_cast<size_t>(bh) * a.S * dk;
   const float scale_t = static_cast<float>(static_cast<half_t>(a.scale));
-  const float cscale = 1.4426950408889634f / scale_t;  // log2(e) / scale
-  const float lazy = 8.0f / cscale;                     // 2^8 in p, in units of q·k
+  // the scores' unit: q·k, or the rounded and masked score
+  const float cscale = MODE == kMasked ? 1.4426950408889634f : 1.4426950408889634f / scale_t;
+  const float lazy = 8.0f / cscale;  // 2^8 in p
   const int qw = q0 + wave * 32;     // first query of this wave
   const int myq = qw + (lane & 31);  // this lane's query
   const int hi = lane >> 5;          // which half of the wave
@@ -839,38 +858,57 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pipe_kernel(AttnArgs a) {
   half8 qb[KS];
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks)
-    qb[ks] = myq < S ? *reinterpret_cast<const half8*>(Qg + static_cast<size_t>(myq) * DK + ks * 16 + hi * 8)
-                     : z8;
-  const int kend = base + min(q0 + kFQ, S);  // keys of the workgroup's last query
-  const int nt = (kend + kFK - 1) / kFK;     // key tiles of the workgroup
-  const int ntw = qw < S ? (base + min(qw + 31, S - 1)) / kFK + 1 : 0;  // tiles this wave reads
+    qb[ks] = myq < S && (!PAD || ks * 16 + hi * 8 < dk)
+                 ? *reinterpret_cast<const half8*>(Qg + static_cast<size_t>(myq) * dk + ks * 16 + hi * 8)
+                 : z8;
+  const int kend = MODE == kCausal ? base + min(q0 + kFQ, S) : S;  // keys of the workgroup's last query
+  const int nt = (kend + kFK - 1) / kFK;                           // key tiles of the workgroup
+  // tiles this wave reads
+  int ntw = qw >= S ? 0 : MODE == kCausal ? (base + min(qw + 31, S - 1)) / kFK + 1 : nt;
+  // this wave's first masked tile ends past here
+  int unmasked = MODE == kCausal ? base + qw : kend - 1;
+  // (kept as vector values, as the causal ones are: scalar tests fold into each other and into
+  // the loop's, the bodies merge, and head dim 128 spills a hundred registers)
+  if constexpr (MODE != kCausal) asm volatile("" : "+v"(ntw), "+v"(unmasked));
 
   // K and V through buffer loads: bytes past the last key (kend rows) read as zero, so
   // a tile needs no bounds tests (the causal mask removes those keys), and a tile's
   // offset is a scalar added to a fixed per-thread offset.
-  const int kv_bytes = kend * DK * static_cast<int>(sizeof(half_t));
+  const int kv_bytes = kend * dk * static_cast<int>(sizeof(half_t));
   const __amdgpu_buffer_rsrc_t kres =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(Kg), static_cast<short>(0), kv_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t vres =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(Vg), static_cast<short>(0), kv_bytes, 0x00020000);
-  constexpr int kTileBytes = kFK * DK * 2;
-  const int koff = (tid / VG) * DK * 2 + (tid % VG) * 16;  // piece i: + i·4096 bytes (256/VG keys)
-  const int voff = 2 * (tid & 31) * DK * 2 + (tid >> 5) * 16;
-  half8 kn[CH], vn[CH];
+  const int kTileBytes = kFK * dk * 2;
+  // Piece i of K: chunk tid + 256 i of the tile. With 256 a whole number of rows (every DK but
+  // 96) the pieces are a fixed distance apart; pieces past dk read past the end (zero).
+  constexpr int kPast = 0x7ffffff0;
+  int koff[CH], voff[VI];
+#pragma unroll
+  for (int i = 0; i < CH; ++i) {
+    const int c = tid + 256 * i, d8 = (c % VG) * 8;
+    koff[i] = PAD && d8 >= dk ? kPast : (c / VG) * dk * 2 + d8 * 2;
+  }
+#pragma unroll
+  for (int i = 0; i < VI; ++i) {
+    const int grp = (tid >> 5) + 8 * i;
+    voff[i] = grp >= VG || (PAD && grp * 8 >= dk) ? kPast : 2 * (tid & 31) * dk * 2 + grp * 16;
+  }
+  half8 kn[CH], vn[2 * VI];
   auto fetch_k = [&](int t, half8 (&dst)[CH]) {
 #pragma unroll
     for (int i = 0; i < CH; ++i)
-      dst[i] = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(kres, koff, t * kTileBytes + i * 4096, 0));
+      dst[i] = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(kres, koff[i], t * kTileBytes, 0));
   };
   // V as key pairs (keys 2p, 2p + 1 of the same 8 dims, p = tid % 32): the transposed
   // store is one 4-byte word per dim, 32 lanes covering a 128-byte row segment of Vt
   auto fetch_v = [&](int t) {
 #pragma unroll
-    for (int i = 0; i < CH / 2; ++i)
+    for (int i = 0; i < VI; ++i)
 #pragma unroll
       for (int u = 0; u < 2; ++u)
         vn[2 * i + u] = __builtin_bit_cast(
-            half8, __builtin_amdgcn_raw_buffer_load_b128(vres, voff + u * DK * 2 + i * 128, t * kTileBytes, 0));
+            half8, __builtin_amdgcn_raw_buffer_load_b128(vres, voff[i], t * kTileBytes + u * dk * 2, 0));
   };
   auto put_k = [&](auto buf_c, const half8 (&src)[CH]) {
     constexpr int buf = decltype(buf_c)::value;
@@ -884,8 +922,9 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pipe_kernel(AttnArgs a) {
   auto put_v = [&](auto buf_c) {
     constexpr int buf = decltype(buf_c)::value;
 #pragma unroll
-    for (int i = 0; i < CH / 2; ++i) {
+    for (int i = 0; i < VI; ++i) {
       const int grp = (tid >> 5) + 8 * i, key = 2 * (tid & 31);
+      if (VG % 8 != 0 && grp >= VG) continue;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const half2v pr = {vn[2 * i][e], vn[2 * i + 1][e]};
@@ -918,18 +957,53 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pipe_kernel(AttnArgs a) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[t][r] = 0.f;
 
-  // Masking of tile t's scores (keys after the query: −∞), their maximum, and the
+  // The mask of tile t for this lane's query, by the keys of its score registers (4
+  // consecutive keys a load; a column past the last key reads the last one, see prep).
+  const half_t* __restrict__ mrow =
+      MODE == kMasked ? static_cast<const half_t*>(a.mask) + static_cast<size_t>(min(myq, S - 1)) * S : nullptr;
+  const bool mvec = MODE == kMasked && (S & 3) == 0 && (reinterpret_cast<uintptr_t>(a.mask) & 7) == 0;
+  auto fetch_mask = [&](int key, half4& mk) {
+    if (mvec) {
+      mk = *reinterpret_cast<const half4*>(mrow + min(key, S - 4));
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) mk[e] = mrow[min(key + e, S - 1)];
+    }
+  };
+  const float rscale = 1.0f / scale_t;
+  // rnd(rnd(x) / scale) with the quotient of fp32 division: the product with the reciprocal,
+  // corrected by its remainder
+  auto round_score = [&](float x) {
+    const float n = static_cast<float>(static_cast<half_t>(x));
+    const float q = n * rscale;
+    const float f = __builtin_fmaf(__builtin_fmaf(-q, scale_t, n), rscale, q);
+    return static_cast<half_t>(__builtin_isfinite(n) ? f : n);
+  };
+  // Masking of tile t's scores (keys after the query or past the last: −∞), their maximum, and the
   // reference point the tile's probabilities will use. A key tile past the sequence's
   // last key never reaches here (kend bounds the tiles), and key 0 precedes every
   // query, so the reference point is finite from the first tile on.
   auto prep = [&](auto mask_c, int t, floatx16 (&s)[2]) {
+    if constexpr (MODE == kMasked) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        half4 mk[4];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) fetch_mask(t * kFK + 32 * u + 8 * g + 4 * hi, mk[g]);
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          s[u][r] = static_cast<float>(round_score(s[u][r]) + mk[r >> 2][r & 3]);
+        if constexpr (DK > 64) __builtin_amdgcn_sched_barrier(0);
+      }
+    }
     if constexpr (decltype(mask_c)::value) {
+      const int last = MODE == kCausal ? qpos : kend - 1;
 #pragma unroll
       for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int key = t * kFK + u * 32 + 8 * (r >> 2) + 4 * hi + (r & 3);
-          if (key > qpos) s[u][r] = -INFINITY;
+          if (key > last) s[u][r] = -INFINITY;
         }
     }
     float mloc = s[0][0];
@@ -943,7 +1017,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pipe_kernel(AttnArgs a) {
     grow = __any(mx > m + lazy);
     mnew = grow ? mx : m;
   };
-  auto masked = [&](int t) { return (t + 1) * kFK - 1 > base + qw; };
+  auto masked = [&](int t) { return (t + 1) * kFK - 1 > unmasked; };
 
   // One tile's softmax and P·V, with the next tile's scores (NEXT) beside them. PAR is
   // the tile's parity: its V sits in buffer PAR, the next tile's K in buffer PAR ^ 1
@@ -956,7 +1030,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pipe_kernel(AttnArgs a) {
     constexpr int PAR = decltype(par_c)::value;
     constexpr bool NEXT = decltype(next_c)::value;
     if (grow) {
-      const float alpha = __builtin_amdgcn_exp2f((m - mnew) * cscale);
+      float alpha = __builtin_amdgcn_exp2f((m - mnew) * cscale);
+      if (MODE == kMasked && mnew == -INFINITY) alpha = 1.f;  // nothing summed yet
       l *= alpha;
 #pragma unroll
       for (int t = 0; t < OT; ++t)
@@ -964,40 +1039,69 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pipe_kernel(AttnArgs a) {
         for (int r = 0; r < 16; ++r) o[t][r] *= alpha;
     }
     m = mnew;
+    // (instructions kept in the written order where moved ones cost registers that are not
+    // there: spills)
+    constexpr bool kPin = EXACT && (DK > 64 || MODE == kMasked);
+    if constexpr (kPin) __builtin_amdgcn_sched_barrier(0);
     if constexpr (NEXT) scores(std::integral_constant<int, PAR ^ 1>{}, nxt);
+    if constexpr (kPin) __builtin_amdgcn_sched_barrier(0);
     const float nmx = -m * cscale;
+    // (a masked score may be of the type's lowest value: the difference is formed first)
+    const float mref = MODE == kMasked && m == -INFINITY ? 0.f : m;
+    auto prob = [&](float s) {
+      if constexpr (MODE == kMasked)
+        return __builtin_amdgcn_exp2f((s - mref) * cscale);
+      else
+        return __builtin_amdgcn_exp2f(__builtin_fmaf(s, cscale, nmx));
+    };
     const half2v ones = {static_cast<_Float16>(1.0f), static_cast<_Float16>(1.0f)};
-    half8 pb[4];
+    half8 pb[4], pl[4];
+    auto probs = [&](int blk) {  // of the tile's 16-key block blk
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int jj = 0; jj < 8; jj += 2) {
-          const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(cur[t][8 * kb + jj], cscale, nmx));
-          const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(cur[t][8 * kb + jj + 1], cscale, nmx));
-          const half2v pp = {static_cast<_Float16>(p0), static_cast<_Float16>(p1)};
-          l = __builtin_amdgcn_fdot2(pp, ones, l, false);
-          pb[2 * t + kb][jj] = pp[0];
-          pb[2 * t + kb][jj + 1] = pp[1];
-        }
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
-        const int kblk = t * 32 + kb * 16 + 4 * hi;
-#pragma unroll
-        for (int ot = 0; ot < OT; ++ot) {
-          const half_t* vrow = &Vt[PAR][ot * 32 + (lane & 31)][kblk];
-          half8 va;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            va[e] = vrow[e];
-            va[4 + e] = vrow[8 + e];
-          }
-          o[ot] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pb[2 * t + kb], o[ot], 0, 0, 0);
+      for (int jj = 0; jj < 8; jj += 2) {
+        const float p0 = prob(cur[blk >> 1][8 * (blk & 1) + jj]);
+        const float p1 = prob(cur[blk >> 1][8 * (blk & 1) + jj + 1]);
+        const half2v pp = {static_cast<_Float16>(p0), static_cast<_Float16>(p1)};
+        l = __builtin_amdgcn_fdot2(pp, ones, l, false);
+        pb[blk][jj] = pp[0];
+        pb[blk][jj + 1] = pp[1];
+        if constexpr (EXACT) {
+          const half2v pr = {static_cast<_Float16>(p0 - static_cast<float>(pp[0])),
+                             static_cast<_Float16>(p1 - static_cast<float>(pp[1]))};
+          l = __builtin_amdgcn_fdot2(pr, ones, l, false);
+          pl[blk][jj] = pr[0];
+          pl[blk][jj + 1] = pr[1];
         }
       }
+    };
+    auto add_pv = [&](int blk) {
+      const int kblk = (blk >> 1) * 32 + (blk & 1) * 16 + 4 * hi;
+#pragma unroll
+      for (int ot = 0; ot < OT; ++ot) {
+        const half_t* vrow = &Vt[PAR][ot * 32 + (lane & 31)][kblk];
+        half8 va;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          va[e] = vrow[e];
+          va[4 + e] = vrow[8 + e];
+        }
+        o[ot] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pb[blk], o[ot], 0, 0, 0);
+        if constexpr (EXACT) o[ot] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pl[blk], o[ot], 0, 0, 0);
+      }
+    };
+    if constexpr (EXACT) {  // block by block: both parts of all four at once do not fit
+#pragma unroll
+      for (int blk = 0; blk < 4; ++blk) {
+        probs(blk);
+        add_pv(blk);
+        if constexpr (kPin) __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+#pragma unroll
+      for (int blk = 0; blk < 4; ++blk) probs(blk);
+#pragma unroll
+      for (int blk = 0; blk < 4; ++blk) add_pv(blk);
+    }
     if constexpr (NEXT) prep(mask_next_c, j + 1, nxt);
   };
   auto iter = [&](auto par_c, int j, floatx16 (&cur)[2], floatx16 (&nxt)[2]) {
@@ -1043,24 +1147,26 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pipe_kernel(AttnArgs a) {
   l += __shfl_xor(l, 32, 64);
   if (myq < S) {
     const float inv = 1.f / l;
-    const int hd = a.H * DK;
+    const int hd = a.H * dk;
     const size_t row = (a.row_start ? a.row_start[b] : static_cast<size_t>(b) * S) + myq;
-    half_t* out = static_cast<half_t*>(a.out) + row * hd + h * DK;
+    half_t* out = static_cast<half_t*>(a.out) + row * hd + h * dk;
 #pragma unroll
     for (int ot = 0; ot < OT; ++ot)
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        out[ot * 32 + 8 * (r >> 2) + 4 * hi + (r & 3)] = static_cast<half_t>(o[ot][r] * inv);
+      for (int r = 0; r < 16; ++r) {
+        const int d = ot * 32 + 8 * (r >> 2) + 4 * hi + (r & 3);
+        if (!PAD || d < dk) out[d] = static_cast<half_t>(o[ot][r] * inv);
+      }
   }
 }
 
 
-// fp32 causal prefill on MFMA 32×32×2 (head dims 64 and 128): 4 waves × 32 queries per
-// block, key tiles of 64 through LDS. Each wave computes Sᵀ = K·Qᵀ (keys as rows) so
-// that lane l and lane l ^ 32 own query l % 32: the online-softmax state is per lane,
-// and Oᵀ = Vᵀ·Pᵀ takes the probabilities straight from the registers (lane l supplies
-// key rows f(r) for k = 0 and f(r) + 4 for k = 1 of the 32 × 32 tile, which only
-// reorders the sum). Scores are q·k / scale in fp32 as in attn_prefill_kernel.
+// fp32 prefill on MFMA 32×32×2: 4 waves × 32 queries per block, key tiles of 64 through LDS.
+// Each wave computes Sᵀ = K·Qᵀ (keys as rows) so that lane l and lane l ^ 32 own query
+// l % 32: the online-softmax state is per lane, and Oᵀ = Vᵀ·Pᵀ takes the probabilities
+// straight from the registers (lane l supplies key rows f(r) for k = 0 and f(r) + 4 for
+// k = 1 of the 32 × 32 tile, which only reorders the sum). Scores are q·k / scale in fp32 as
+// in attn_prefill_kernel. MODE and PAD as in attn_prefill_pipe_kernel.
 constexpr int kF32Q = 128, kF32K = 64;
 
 template <int DK>
@@ -1068,10 +1174,11 @@ constexpr size_t f32_mfma_lds() {
   return 2 * kF32K * (DK + 1) * sizeof(float);
 }
 
-template <int DK>
+template <int DK, int MODE, bool PAD>
 __global__ __launch_bounds__(256) void attn_prefill_f32_mfma(AttnArgs a) {
   extern __shared__ float lds[];
   constexpr int P = DK + 1, NJ = DK / 32;
+  const int dk = PAD ? a.dk : DK;
   float* Ks = lds;
   float* Vs = lds + kF32K * P;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, l32 = lane & 31, hi = lane >> 5;
@@ -1082,17 +1189,20 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_mfma(AttnArgs a) {
   const int base = a.pos_base ? a.pos_base[b] : 0;
   const int s = q0 + 32 * w + l32;
   const bool valid = s < S;
-  const int qpos = base + (valid ? s : S - 1);
-  const int kv_end = base + min(S, q0 + kF32Q);                  // keys of the block
-  const int wave_last = base + min(S - 1, q0 + 32 * w + 31);     // last key this wave needs
+  const int sc_row = valid ? s : S - 1;
+  // this lane's last key, the block's end, and the last key this wave needs
+  const int last = MODE == kCausal ? base + sc_row : S - 1;
+  const int kv_end = MODE == kCausal ? base + min(S, q0 + kF32Q) : S;
+  const int wave_last = MODE == kCausal ? base + min(S - 1, q0 + 32 * w + 31) : S - 1;
   const float* __restrict__ K = static_cast<const float*>(a.k) + b * a.kv_stride_b + h * a.kv_stride_h;
   const float* __restrict__ V = static_cast<const float*>(a.v) + b * a.kv_stride_b + h * a.kv_stride_h;
+  const float* __restrict__ mrow =
+      MODE == kMasked ? static_cast<const float*>(a.mask) + static_cast<size_t>(sc_row) * S : nullptr;
   float qr[DK / 2];  // Q[s][2i + hi]: the B operand of Sᵀ
   {
-    const float* qp = static_cast<const float*>(a.q) +
-                      (static_cast<size_t>(bh) * a.S + (valid ? s : S - 1)) * DK + hi;
+    const float* qp = static_cast<const float*>(a.q) + (static_cast<size_t>(bh) * a.S + sc_row) * dk + hi;
 #pragma unroll
-    for (int i = 0; i < DK / 2; ++i) qr[i] = qp[2 * i];
+    for (int i = 0; i < DK / 2; ++i) qr[i] = !PAD || 2 * i + hi < dk ? qp[2 * i] : 0.f;
   }
   floatx16 o[NJ];
 #pragma unroll
@@ -1108,9 +1218,9 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_mfma(AttnArgs a) {
       const int e = threadIdx.x + 256 * i;
       const int r = e / (DK / 4), c = (e - r * (DK / 4)) * 4;
       const floatx4 z = {0.f, 0.f, 0.f, 0.f};
-      const bool ok = k0 + r < kv_end;
-      nk[i] = ok ? *reinterpret_cast<const floatx4*>(K + static_cast<long long>(k0 + r) * DK + c) : z;
-      nv[i] = ok ? *reinterpret_cast<const floatx4*>(V + static_cast<long long>(k0 + r) * DK + c) : z;
+      const bool ok = k0 + r < kv_end && (!PAD || c < dk);
+      nk[i] = ok ? *reinterpret_cast<const floatx4*>(K + static_cast<long long>(k0 + r) * dk + c) : z;
+      nv[i] = ok ? *reinterpret_cast<const floatx4*>(V + static_cast<long long>(k0 + r) * dk + c) : z;
     }
   };
   fetch(0);
@@ -1129,6 +1239,12 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_mfma(AttnArgs a) {
     __syncthreads();
     if (k0 + kF32K < kv_end) fetch(k0 + kF32K);
     if (k0 > wave_last) continue;  // every key of the tile is after this wave's queries
+    float mk[32];
+    if constexpr (MODE == kMasked) {  // in flight beside the scores
+#pragma unroll
+      for (int e = 0; e < 32; ++e)
+        mk[e] = mrow[min(k0 + 32 * (e >> 4) + 8 * ((e & 15) >> 2) + 4 * hi + (e & 3), S - 1)];
+    }
     floatx16 sc[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -1145,20 +1261,24 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_mfma(AttnArgs a) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int key = k0 + 32 * t + 8 * (r >> 2) + 4 * hi + (r & 3);
-        const float v = key <= qpos ? sc[t][r] / a.scale : -INFINITY;
+        float v = sc[t][r] / a.scale;
+        if constexpr (MODE == kMasked) v += mk[16 * t + r];
+        if (key > last) v = -INFINITY;
         sc[t][r] = v;
         mloc = fmaxf(mloc, v);
       }
     mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64));
-    // finite: the first tile holds key 0, which every query sees
+    // finite but for masked scores: the first tile holds key 0, which every query sees
     const float mn = fmaxf(m, mloc);
-    const float alpha = expf(m - mn);
+    if (MODE == kMasked && __all(mn == -INFINITY)) continue;  // nothing to add yet
+    const float mref = MODE == kMasked && mn == -INFINITY ? 0.f : mn;
+    const float alpha = expf(m - mref);
     float lsum = 0.f;
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const float p = expf(sc[t][r] - mn);
+        const float p = expf(sc[t][r] - mref);
         sc[t][r] = p;
         lsum += p;
       }
@@ -1180,12 +1300,15 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_mfma(AttnArgs a) {
   }
   if (valid) {
     const size_t row = (a.row_start ? a.row_start[b] : static_cast<size_t>(b) * a.S) + s;
-    float* out = static_cast<float*>(a.out) + row * a.H * DK + h * DK;
+    float* out = static_cast<float*>(a.out) + row * a.H * dk + h * dk;
     const float inv = 1.f / l;
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) out[32 * j + 8 * (r >> 2) + 4 * hi + (r & 3)] = o[j][r] * inv;
+      for (int r = 0; r < 16; ++r) {
+        const int d = 32 * j + 8 * (r >> 2) + 4 * hi + (r & 3);
+        if (!PAD || d < dk) out[d] = o[j][r] * inv;
+      }
     if (a.lse && hi == 0) a.lse[static_cast<size_t>(bh) * a.S + s] = m + logf(l);
     if (a.m_out && hi == 0) {
       a.m_out[static_cast<size_t>(bh) * a.S + s] = m;
@@ -1194,50 +1317,112 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_mfma(AttnArgs a) {
   }
 }
 
-template <int DK>
-int prefill_f32_mfma(const AttnArgs& a, hipStream_t st) {
+template <int DK, int MODE, bool PAD>
+int prefill_f32_mfma_launch(const AttnArgs& a, hipStream_t st) {
   constexpr size_t lds = f32_mfma_lds<DK>();
   static bool attr = false;
   if (!attr) {
-    NML_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_prefill_f32_mfma<DK>),
+    NML_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_prefill_f32_mfma<DK, MODE, PAD>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
     attr = true;
   }
   dim3 grid((a.S + kF32Q - 1) / kF32Q, a.B * a.H);
-  attn_prefill_f32_mfma<DK><<<grid, 256, lds, st>>>(a);
+  attn_prefill_f32_mfma<DK, MODE, PAD><<<grid, 256, lds, st>>>(a);
   NML_LAUNCHED();
   return 0;
 }
 
+AttnMode attn_mode(const AttnArgs& a) { return !a.full ? kCausal : a.mask ? kMasked : kFull; }
+
+// Whether the matrix-core kernels take the call: head dims up to 128 in whole 16-byte pieces,
+// every row 16-byte aligned.
+template <typename T>
+bool prefill_mfma_applies(const AttnArgs& a) {
+  constexpr int vec = 16 / sizeof(T);
+  return a.dk <= 128 && a.dk % vec == 0 && a.kv_stride_b % vec == 0 && a.kv_stride_h % vec == 0 &&
+         ((reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.k) |
+           reinterpret_cast<uintptr_t>(a.v)) & 15) == 0;
+}
+
+template <int DK, int MODE>
+int prefill_f32_mfma(const AttnArgs& a, hipStream_t st) {
+  return a.dk == DK ? prefill_f32_mfma_launch<DK, MODE, false>(a, st)
+                    : prefill_f32_mfma_launch<DK, MODE, true>(a, st);
+}
+
+template <int MODE>
+int prefill_f32_mode(const AttnArgs& a, hipStream_t st) {
+  if (a.dk <= 32) return prefill_f32_mfma<32, MODE>(a, st);
+  if (a.dk <= 64) return prefill_f32_mfma<64, MODE>(a, st);
+  if (a.dk <= 96) return prefill_f32_mfma<96, MODE>(a, st);
+  return prefill_f32_mfma<128, MODE>(a, st);
+}
+
+template <int DK, int MODE, bool PAD, bool EXACT>
+int prefill_pipe_launch(const AttnArgs& a, hipStream_t st) {
+  attn_prefill_pipe_kernel<DK, MODE, PAD, EXACT>
+      <<<dim3((a.S + kFQ - 1) / kFQ, a.B * a.H), 256, 0, st>>>(a);
+  NML_LAUNCHED();
+  return 0;
+}
+
+template <int DK, int MODE>
+int prefill_pipe(const AttnArgs& a, hipStream_t st) {
+  constexpr bool exact = MODE != kCausal || (DK != 64 && DK != 128);
+  if (a.dk != DK) return prefill_pipe_launch<DK, MODE, true, true>(a, st);
+  return prefill_pipe_launch<DK, MODE, false, exact>(a, st);
+}
+
+template <int MODE>
+int prefill_pipe_mode(const AttnArgs& a, hipStream_t st) {
+  if (a.dk <= 32) return prefill_pipe<32, MODE>(a, st);
+  if (a.dk <= 64) return prefill_pipe<64, MODE>(a, st);
+  if (a.dk <= 96) return prefill_pipe<96, MODE>(a, st);
+  return prefill_pipe<128, MODE>(a, st);
+}
+
+// The scalar kernel of head dims 8, 16 and 32 (and, for calls the matrix cores do not take, 64
+// and 128).
 template <typename T, int DK>
-int prefill_typed(const AttnArgs& a, hipStream_t st) {
-  if (a.full) {  // non-causal / masked: the scalar kernel only
-    NML_REQUIRE(!a.pos_base && !a.seq_len && !a.row_start,
-                "attention: non-causal attention takes dense rows from position 0");
-    dim3 grid((a.S + kTile - 1) / kTile, a.B * a.H);
-    attn_prefill_kernel<T, DK><<<grid, 64, 0, st>>>(a);
-    NML_LAUNCHED();
-    return 0;
-  }
-  if constexpr (sizeof(T) == 4 && (DK == 64 || DK == 128)) {
-    if (!std::getenv("NIMBLEML_ATTN_F32_SCALAR")) return prefill_f32_mfma<DK>(a, st);
-  }
-  if constexpr (sizeof(T) == 2 && (DK == 64 || DK == 128)) {
-    dim3 grid((a.S + kFQ - 1) / kFQ, a.B * a.H);
-    // fp16-rounded scores where the backward recomputes them from the statistics
-    // The pipelined kernel's buffer loads take a 32-bit byte range per (row, head): a
-    // cache row block past 2 GiB (kv_stride_h elements) takes the other kernel.
-    const bool ranged = a.kv_stride_h * static_cast<long long>(sizeof(half_t)) < (1LL << 31);
-    if (a.lse || a.m_out || !ranged)
-      attn_prefill_mfma_kernel<DK><<<grid, 256, 0, st>>>(a);
-    else
-      attn_prefill_pipe_kernel<DK><<<grid, 256, 0, st>>>(a);
-    NML_LAUNCHED();
-    return 0;
-  }
+int prefill_scalar(const AttnArgs& a, hipStream_t st) {
   dim3 grid((a.S + kTile - 1) / kTile, a.B * a.H);
   attn_prefill_kernel<T, DK><<<grid, 64, 0, st>>>(a);
   NML_LAUNCHED();
+  return 0;
+}
+
+// Matrix cores where the call allows it. fp16 calls that keep the softmax statistics take
+// fp16-rounded scores, as the backward recomputes them: head dims 64 and 128 causal have such a
+// kernel. (The pipelined kernel's buffer loads take a 32-bit byte range per (row, head): a
+// cache row block past 2 GiB takes another kernel.)
+template <typename T>
+int prefill_matrix(const AttnArgs& a, hipStream_t st, bool* taken) {
+  *taken = true;
+  const AttnMode mode = attn_mode(a);
+  if (prefill_mfma_applies<T>(a)) {
+    if constexpr (sizeof(T) == 4) {
+      if (!std::getenv("NIMBLEML_ATTN_F32_SCALAR")) {
+        if (mode == kCausal) return prefill_f32_mode<kCausal>(a, st);
+        return mode == kFull ? prefill_f32_mode<kFull>(a, st) : prefill_f32_mode<kMasked>(a, st);
+      }
+    } else {
+      const bool ranged = a.kv_stride_h * static_cast<long long>(sizeof(half_t)) < (1LL << 31);
+      if (!a.lse && !a.m_out && ranged) {
+        if (mode == kCausal) return prefill_pipe_mode<kCausal>(a, st);
+        return mode == kFull ? prefill_pipe_mode<kFull>(a, st) : prefill_pipe_mode<kMasked>(a, st);
+      }
+      if (mode == kCausal && (a.dk == 64 || a.dk == 128)) {
+        const dim3 grid((a.S + kFQ - 1) / kFQ, a.B * a.H);
+        if (a.dk == 64)
+          attn_prefill_mfma_kernel<64><<<grid, 256, 0, st>>>(a);
+        else
+          attn_prefill_mfma_kernel<128><<<grid, 256, 0, st>>>(a);
+        NML_LAUNCHED();
+        return 0;
+      }
+    }
+  }
+  *taken = false;
   return 0;
 }
 
@@ -1273,12 +1458,17 @@ int prefill_quad(const AttnArgs& a, hipStream_t st) {
 
 template <typename T>
 int prefill_dk(const AttnArgs& a, hipStream_t st) {
+  NML_REQUIRE(!a.full || (!a.pos_base && !a.seq_len && !a.row_start),
+              "attention: non-causal attention takes dense rows from position 0");
+  bool taken = false;
+  NML_TRY(prefill_matrix<T>(a, st, &taken));
+  if (taken) return 0;
   switch (a.dk) {
-    case 8: return prefill_typed<T, 8>(a, st);
-    case 16: return prefill_typed<T, 16>(a, st);
-    case 32: return prefill_typed<T, 32>(a, st);
-    case 64: return prefill_typed<T, 64>(a, st);
-    case 128: return prefill_typed<T, 128>(a, st);
+    case 8: return prefill_scalar<T, 8>(a, st);
+    case 16: return prefill_scalar<T, 16>(a, st);
+    case 32: return prefill_scalar<T, 32>(a, st);
+    case 64: return prefill_scalar<T, 64>(a, st);
+    case 128: return prefill_scalar<T, 128>(a, st);
   }
   // other head dims: four lanes per query, dims padded to 32, 64, 128 or 256
   if (a.dk <= 32) return prefill_quad<T, 8>(a, st);
