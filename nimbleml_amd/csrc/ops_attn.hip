@@ -805,11 +805,12 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_kernel(AttnArgs a) {
 //
 // MODE: causal; full (every key); or full with an additive (S, S) mask. PAD: the head dim
 // a.dk (a multiple of 8) is below DK: dims past it read as zero and are not stored. EXACT: the
-// probabilities enter P·V as two fp16 parts (22 bits) and two products, for the calls that
-// took float32 probabilities from the scalar kernels before (every one but causal head dims
-// 64 and 128); their scores stay float32 accumulators, except that a masked score is rounded
-// as the reference's fp16 ops round it, rnd(rnd(rnd(q·k) / scale) + mask): a mask of the
-// type's lowest value must absorb the score. A tile whose keys are all −∞ for a query leaves
+// probabilities enter P·V as two fp16 parts (22 bits) and two products, which leaves them the
+// float32 precision of the scalar kernels (every call but causal head dims 64 and 128). The
+// scores stay float32 accumulators at head dims 64 and 128; at others, and masked, they are
+// rounded as the reference's fp16 ops round them, rnd(rnd(rnd(q·k) / scale) + mask): a mask of
+// the type's lowest value must absorb the score, and the logits of small models are held
+// against the fp16 reference's. A tile whose keys are all −∞ for a query leaves
 // its reference point at −∞ and adds nothing; a query with no other key gives NaN, as a
 // softmax over nothing does.
 // 4 × 16 heads × 1024 keys of 64 dims, every key: the scalar kernel's 826 µs fell to 42 (410
@@ -847,8 +848,9 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pipe_kernel(AttnArgs a) {
   const half_t* __restrict__ Vg = static_cast<const half_t*>(a.v) + b * a.kv_stride_b + h * a.kv_stride_h;
   const half_t* __restrict__ Qg = static_cast<const half_t*>(a.q) + static_cast<size_t>(bh) * a.S * dk;
   const float scale_t = static_cast<float>(static_cast<half_t>(a.scale));
-  // the scores' unit: q·k, or the rounded and masked score
-  const float cscale = MODE == kMasked ? 1.4426950408889634f : 1.4426950408889634f / scale_t;
+  // the scores' unit: q·k, or the rounded (and masked) score
+  constexpr bool kRounded = MODE == kMasked || PAD || (DK != 64 && DK != 128);
+  const float cscale = kRounded ? 1.4426950408889634f : 1.4426950408889634f / scale_t;
   const float lazy = 8.0f / cscale;  // 2^8 in p
   const int qw = q0 + wave * 32;     // first query of this wave
   const int myq = qw + (lane & 31);  // this lane's query
@@ -984,15 +986,20 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pipe_kernel(AttnArgs a) {
   // last key never reaches here (kend bounds the tiles), and key 0 precedes every
   // query, so the reference point is finite from the first tile on.
   auto prep = [&](auto mask_c, int t, floatx16 (&s)[2]) {
-    if constexpr (MODE == kMasked) {
+    if constexpr (kRounded) {
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         half4 mk[4];
+        if constexpr (MODE == kMasked) {
 #pragma unroll
-        for (int g = 0; g < 4; ++g) fetch_mask(t * kFK + 32 * u + 8 * g + 4 * hi, mk[g]);
+          for (int g = 0; g < 4; ++g) fetch_mask(t * kFK + 32 * u + 8 * g + 4 * hi, mk[g]);
+        }
 #pragma unroll
-        for (int r = 0; r < 16; ++r)
-          s[u][r] = static_cast<float>(round_score(s[u][r]) + mk[r >> 2][r & 3]);
+        for (int r = 0; r < 16; ++r) {
+          half_t v = round_score(s[u][r]);
+          if constexpr (MODE == kMasked) v = v + mk[r >> 2][r & 3];
+          s[u][r] = static_cast<float>(v);
+        }
         if constexpr (DK > 64) __builtin_amdgcn_sched_barrier(0);
       }
     }
