@@ -581,9 +581,188 @@ __device__ int find_nth(int V, int j, FP pred, Shared& sh) {
   return sh.found_index;
 }
 
+// ---------------------------------------------------------------- top-p from registers
+// Top-p (with or without top-k) with the row's probabilities in registers: thread t holds
+// elements t + 1024 j (E of them), computed once, where the general path forms each again in
+// every one of its ~20 passes. Each "first position of the descending order whose running
+// mass exceeds a target" is one pass over a histogram of counts and masses on the leading
+// bits of the key below the largest key (2^kBinBits bins of 1/128 of an octave, the elements
+// spread over hundreds of them, so the LDS atomics seldom meet), a scan of the bins, and the
+// walk order inside the bin that the target falls into. Sums over the row are taken as the
+// general path takes them. Declines (the general path then runs) when that bin holds more
+// than kBinCand elements, as a row of equal or of no logits does.
+// 32 rows of 32000 fp16 logits, top-p 0.9: 377 µs on the general path (about 20 passes of
+// exponentials and divisions, and LDS atomics on the few bins that the leading byte of a
+// probability can fall into), 94 here.
+constexpr int kBinBits = 12, kBins = 1 << kBinBits, kBinShift = 16, kBinCand = 1024;
+
+struct BinCand {
+  uint32_t key;
+  int index;
+  double w;
+};
+struct BinWork {  // (the row cache's LDS)
+  double mass[kBins];
+  int cnt[kBins];
+  BinCand cand[kBinCand];
+  int n, bin, last;
+  double before;
+  unsigned long long best, least;
+};
+
+__device__ __forceinline__ float key_value(uint32_t k) {
+  return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
+}
+
+// The first element of the walk (key descending, then index descending) over the elements with
+// in(j) whose inclusive running weight exceeds target; the walk's last if none does. top: a
+// key no element exceeds. False: declined.
+template <int E, typename FK, typename FW, typename FI>
+__device__ bool walk_to(uint32_t top, double target, FK key_of, FW weight, FI in, Shared& sh, BinWork& bw,
+                        uint32_t* key, int* index) {
+  const int tid = threadIdx.x;
+  __syncthreads();  // the previous walk's readers are done
+  for (int i = tid; i < kBins; i += kThreads) {
+    bw.mass[i] = 0.0;
+    bw.cnt[i] = 0;
+  }
+  if (tid == 0) {
+    bw.n = 0;
+    bw.bin = kBins;
+    bw.last = -1;
+    bw.best = 0ull;
+    bw.least = ~0ull;
+  }
+  __syncthreads();
+  auto bin_of = [&](int j) { return static_cast<int>(min((top - key_of(j)) >> kBinShift, kBins - 1u)); };
+#pragma unroll
+  for (int j = 0; j < E; ++j)
+    if (in(j)) {
+      const int b = bin_of(j);
+      atomicAdd(&bw.cnt[b], 1);
+      atomicAdd(&bw.mass[b], weight(j));
+    }
+  __syncthreads();
+  constexpr int PB = kBins / kThreads;
+  double m[PB], own = 0.0, total = 0.0;
+#pragma unroll
+  for (int e = 0; e < PB; ++e) own += m[e] = bw.mass[PB * tid + e];
+  double cum = block_excl_scan_d(own, &total, sh), cum0[PB];
+#pragma unroll
+  for (int e = 0; e < PB; ++e) {
+    const int b = PB * tid + e;
+    cum0[e] = cum;
+    cum += m[e];
+    if (bw.cnt[b] > 0) {
+      if (cum > target) atomicMin(&bw.bin, b);
+      atomicMax(&bw.last, b);
+    }
+  }
+  __syncthreads();
+  const int bin = bw.bin < kBins ? bw.bin : bw.last;
+  if (bin < 0) return false;
+  if (bin / PB == tid) {
+#pragma unroll
+    for (int e = 0; e < PB; ++e)
+      if (bin % PB == e) bw.before = cum0[e];
+  }
+#pragma unroll
+  for (int j = 0; j < E; ++j)
+    if (in(j) && bin_of(j) == bin) {
+      const int at = atomicAdd(&bw.n, 1);
+      if (at < kBinCand) bw.cand[at] = BinCand{key_of(j), tid + kThreads * j, weight(j)};
+    }
+  __syncthreads();
+  const int n = bw.n;
+  if (n > kBinCand) return false;
+  if (tid < n) {
+    const BinCand me = bw.cand[tid];
+    double run = 0.0;
+    for (int c = 0; c < n; ++c) {
+      const BinCand o = bw.cand[c];
+      if (o.key > me.key || (o.key == me.key && o.index >= me.index)) run += o.w;
+    }
+    const unsigned long long code = (static_cast<unsigned long long>(me.key) << 32) | static_cast<uint32_t>(me.index);
+    if (bw.before + run > target) atomicMax(&bw.best, code);
+    atomicMin(&bw.least, code);
+  }
+  __syncthreads();
+  const unsigned long long found = bw.best ? bw.best : bw.least;
+  *key = static_cast<uint32_t>(found >> 32);
+  *index = static_cast<int>(found & 0xffffffffu);
+  return true;
+}
+
+template <typename T, int E>
+__device__ int sample_topp_regs(const Row<T>& row, int k, double top_p, double u, Shared& sh, BinWork& bw) {
+  const int tid = threadIdx.x, V = row.V;
+  float x[E];
+  float mx = -INFINITY;
+#pragma unroll
+  for (int j = 0; j < E; ++j) {
+    const int i = tid + kThreads * j;
+    x[j] = i < V ? row.scaled(i) : -INFINITY;
+    mx = fmaxf(mx, x[j]);
+  }
+  mx = block_max_f(mx, sh);
+  auto held = [&](int j) { return tid + kThreads * j < V; };
+  if (k > 0) {  // the k-th largest: the walk by count
+    uint32_t tk;
+    int at;
+    if (!walk_to<E>(fkey(mx), k - 0.5, [&](int j) { return fkey(x[j]); }, [](int) { return 1.0; }, held, sh, bw,
+                    &tk, &at))
+      return -1;
+    const float thresh = key_value(tk);
+#pragma unroll
+    for (int j = 0; j < E; ++j) x[j] = x[j] < thresh ? -1e9f : x[j];
+  }
+  float se = 0.f;
+#pragma unroll
+  for (int j = 0; j < E; ++j)
+    if (held(j)) {
+      x[j] = expf(x[j] - mx);
+      se += x[j];
+    }
+  se = block_sum_f(se, sh);
+#pragma unroll
+  for (int j = 0; j < E; ++j) x[j] = held(j) ? x[j] / se : 0.f;  // x now holds the probabilities
+  auto keyp = [&](int j) { return fkey(x[j]); };
+  const uint32_t top = fkey(1.0f / se);  // expf(0) / se, the largest probability
+  uint32_t tau;
+  int cut;
+  if (!walk_to<E>(top, top_p, keyp, [&](int j) { return static_cast<double>(x[j]); }, held, sh, bw, &tau, &cut))
+    return -1;
+  // kept: what precedes the cut in the walk; nothing does: the cut alone
+  auto kept = [&](int j) {
+    return held(j) && (keyp(j) > tau || (keyp(j) == tau && tid + kThreads * j > cut));
+  };
+  float ks = 0.f;
+  bool any = false;
+#pragma unroll
+  for (int j = 0; j < E; ++j)
+    if (kept(j)) {
+      ks += x[j];
+      any = true;
+    }
+  ks = block_sum_f(ks, sh);
+  if (!__syncthreads_or(any)) return cut;
+  double tq = 0.0, total = 0.0;
+#pragma unroll
+  for (int j = 0; j < E; ++j)
+    if (kept(j)) tq += static_cast<double>(x[j] / ks);
+  block_excl_scan_d(tq, &total, sh);
+  uint32_t t2;
+  int chosen;
+  if (!walk_to<E>(top, u * total, keyp, [&](int j) { return static_cast<double>(x[j] / ks); }, kept, sh, bw, &t2,
+                  &chosen))
+    return -1;
+  return chosen;
+}
+
 // Logits rows up to this size (V ≤ 51,456 fp16 entries) are staged in LDS once, so the
 // selection passes re-read LDS rather than HBM/L2.
 constexpr int kRowCacheBytes = 100 * 1024 + 512;
+static_assert(sizeof(BinWork) <= kRowCacheBytes, "the top-p walk works in the row cache");
 
 template <typename T>
 __global__ __launch_bounds__(kThreads) void sample_kernel(SampleArgs a) {
@@ -628,6 +807,13 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(SampleArgs a) {
   if constexpr (sizeof(T) == 2) {
     if (sampled && use_k && !use_p && sample_regs_applies(row, k_eff))
       chosen = sample_topk_regs(row, k_eff, u, sh, s_cand, s_candx);
+  }
+  if (sampled && use_p && V <= 50 * kThreads) {
+    BinWork& bw = *reinterpret_cast<BinWork*>(s_row);
+    const int k = use_k ? k_eff : 0;
+    chosen = V <= 32 * kThreads ? sample_topp_regs<T, 32>(row, k, static_cast<double>(a.top_p), u, sh, bw)
+                                : sample_topp_regs<T, 50>(row, k, static_cast<double>(a.top_p), u, sh, bw);
+    __syncthreads();
   }
   if (chosen < 0) {
     // The selection passes re-read the row many times: with room for it, stage it in LDS
