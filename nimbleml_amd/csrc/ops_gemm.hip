@@ -8,8 +8,9 @@
 //    (v_mfma_f32_32x32x16_f16, K=64 per LDS stage). Next stage prefetched into registers
 //    while the current one is multiplied.
 //  * gemm_f32: every float32 value split into three bf16 parts (gemm_split.hpp).
-//  * gemv: M ≤ 8 activation rows (decode). One wave per output row (or four),
-//    16-byte loads along K, fp32 accumulation, wave-reduced.
+//  * gemv: one activation row (decode), or up to 8 short ones. One wave per output row (or four), 16-byte loads
+//    along K, fp32 accumulation, wave-reduced.
+//  * rows: 2 … 8 rows (float32: up to 64), MFMA 16×16 tiles, K split over a workgroup's waves.
 //  * skinny_f16: 8 < M ≤ 64 rows (batched decode), MFMA 16×16×32 with optional split-K
 //    and a fused RMSNorm of x (see its comment).
 #include <cstdlib>
@@ -896,17 +897,145 @@ __global__ __launch_bounds__(256) void gemv_kernel(LinearArgs a) {
     }
 }
 
+// One row; up to 8 of at most 256 values, which one trip of a wave holds (K 256, 8 rows: 4.9 µs
+// here, 5.3 in rows_kernel); two float32 rows against a tied head (N 32000: 28.8 µs here,
+// 30.1 there; at 4 rows 34.0 against 33.1).
+template <typename T>
+bool gemv_applies(const LinearArgs& a) {
+  return a.M == 1 || (a.M <= 8 && a.K <= 256) || (sizeof(T) == 4 && a.M == 2 && a.N >= 8192);
+}
+
 template <typename T, int EPI, int MR>
-int gemv_dispatch_rpw(const LinearArgs& a, hipStream_t st) {
-  if (a.N >= 8192) {
-    const int blocks = (a.N + 15) / 16;
-    gemv_kernel<T, EPI, MR, 4><<<blocks, 256, 0, st>>>(a);
-  } else {
-    const int blocks = (a.N + 3) / 4;
-    gemv_kernel<T, EPI, MR, 1><<<blocks, 256, 0, st>>>(a);
-  }
+int gemv_launch_rows(const LinearArgs& a, hipStream_t st) {
+  if (a.N >= 8192)
+    gemv_kernel<T, EPI, MR, 4><<<(a.N + 15) / 16, 256, 0, st>>>(a);
+  else
+    gemv_kernel<T, EPI, MR, 1><<<(a.N + 3) / 4, 256, 0, st>>>(a);
   NML_LAUNCHED();
   return 0;
+}
+
+template <typename T, int EPI>
+int gemv_launch(const LinearArgs& a, hipStream_t st) {
+  if (a.M <= 1) return gemv_launch_rows<T, EPI, 1>(a, st);
+  if (a.M <= 2) return gemv_launch_rows<T, EPI, 2>(a, st);
+  if (a.M <= 4) return gemv_launch_rows<T, EPI, 4>(a, st);
+  return gemv_launch_rows<T, EPI, 8>(a, st);
+}
+
+// ------------------------------------------------------------------- few rows
+// Decode-sized products on the matrix cores without a workspace. A workgroup owns 16/SP
+// columns (rows of W) × up to 16/SP rows of x; K is divided among its NW waves and, inside
+// each, among SP parts: row (and column) p·16/SP + i of a wave's MFMA tiles holds W row i
+// (x row i) in part p of the wave's k, so the SP blocks on the diagonal of D hold the
+// parts' products (the others are not used). The NW·SP partial tiles are summed through LDS
+// in a fixed order. Every lane loads 16 bytes of a W row and of an x row per k block, U
+// blocks in flight, and feeds them to MFMA 16×16×32 (fp16) or, element j of the four to
+// product j, 16×16×4 (float32): the k order inside a block is the same for both operands,
+// so it only reorders the sum. The row tiles of one column tile follow each other on one
+// XCD, whose L2 holds their W rows.
+// What bounds it: one round trip of the loads and, at float32 with many rows, x's rows from
+// L2 (every column tile reads all of them). SP is for narrow outputs: N = 1024 is 64
+// workgroups of 16 columns, too few to pull 16 MB of W at K = 4096 (8 float32 rows: 17.8 µs
+// with SP 1, 11.8 with 2).
+// It replaces a GEMV of one wave per output (one round trip per 512 k: K 4096, N 1024, 8
+// rows 13.5 → 6.3 µs fp16, 28.5 → 11.8 float32) and 128 × 128 GEMM tiles on a few CUs (48
+// float32 rows: 302 → 20 µs).
+template <typename T, int EPI, int NW, int SP>
+__global__ __launch_bounds__(64 * NW) void rows_kernel(LinearArgs a, int row_tiles, int tiles) {
+  using V = typename Vec16<T>::type;
+  constexpr int VN = Vec16<T>::n, KB = 4 * VN, U = 8, C = 16 / SP;
+  __shared__ float red[NW][16][17];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, g = lane >> 4;
+  const int M = a.M, N = a.N, K = a.K;
+  const int t = row_tiles == 1 ? static_cast<int>(blockIdx.x) : big::xcd_tile(blockIdx.x, tiles);
+  const int n0 = t / row_tiles * C, m0 = t % row_tiles * C;
+  // rows past the last read the last; their products are not stored
+  const T* wp = static_cast<const T*>(a.w) + static_cast<long long>(min(n0 + r % C, N - 1)) * K;
+  const T* xp = static_cast<const T*>(a.x) + static_cast<long long>(min(m0 + r % C, M - 1)) * a.lda;
+  // the output this thread finishes (threads below C²): its bias and residual, in the
+  // operands' round trip
+  const int oi = tid % C, oj = tid / C % C, on = n0 + oi, om = m0 + oj;
+  float bias_v = 0.f, resid_v = 0.f;
+  if constexpr (EPI != EPI_NONE) bias_v = static_cast<float>(static_cast<const T*>(a.bias)[min(on, N - 1)]);
+  if constexpr (EPI == EPI_BIAS_RESID)
+    resid_v = static_cast<float>(
+        static_cast<const T*>(a.resid)[static_cast<size_t>(min(om, M - 1)) * N + min(on, N - 1)]);
+  const int nb = (K + KB - 1) / KB, per = (nb + NW * SP - 1) / (NW * SP);
+  const int b0 = (wave * SP + r / C) * per, b1 = min(nb, b0 + per);  // this lane's blocks
+  V z;
+#pragma unroll
+  for (int e = 0; e < VN; ++e) z[e] = static_cast<T>(0.f);
+  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < per; s += U) {
+    V wv[U], xv[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {  // unconditional loads at clamped places, zeroed past the end
+      const int k = (b0 + s + u) * KB + g * VN;
+      const bool ok = s + u < per && b0 + s + u < b1 && k < K;
+      wv[u] = *reinterpret_cast<const V*>(wp + (ok ? k : 0));
+      xv[u] = *reinterpret_cast<const V*>(xp + (ok ? k : 0));
+      wv[u] = ok ? wv[u] : z;
+      xv[u] = ok ? xv[u] : z;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if constexpr (sizeof(T) == 2) {
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv[u], xv[u], acc, 0, 0, 0);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[u][j], xv[u][j], acc, 0, 0, 0);
+      }
+    }
+  }
+  // D: lane l holds rows 4(l/16) + e (W) of column l%16 (x)
+#pragma unroll
+  for (int e = 0; e < 4; ++e) red[wave][4 * g + e][r] = acc[e];
+  __syncthreads();
+  if (tid >= C * C || om >= M || on >= N) return;
+  float sum = 0.f;
+#pragma unroll
+  for (int w = 0; w < NW; ++w)
+#pragma unroll
+    for (int p = 0; p < SP; ++p) sum += red[w][p * C + oi][p * C + oj];
+  epilogue_with<T, EPI>(a, om, on, sum, bias_v, resid_v);
+}
+
+// fp16: 2 … 8 rows (the skinny kernel takes 9 … 64 where K is a multiple of 128, this one the
+// others of more than 256). float32: up to 16 rows, and more while the output is at most 1024 tiles of 16 × 16:
+// a round of 256 tiles costs 4.8 µs per 1024 of K, the 64 × 64 tile kernel about 20 however
+// few tiles it has (N 4096, K 1024: 64 rows 19.2 µs, 96 rows 26.7 against 21.1; N 1024: 256
+// rows 18.1 against 20.4, 384 rows 25.6 against 20.8; N 32000: 16 rows 41 against 55, 32 rows
+// 70 against 55).
+template <typename T>
+bool rows_applies(const LinearArgs& a) {
+  if (a.ssq_in || a.ssq_out || a.pre_out || a.M < 2) return false;
+  if (sizeof(T) == 2) return a.M <= 8 || (a.M <= 64 && a.K > 256 && a.K % 128 != 0);
+  return a.M <= 16 || ((a.M + 15LL) / 16) * ((a.N + 15LL) / 16) <= 1024;
+}
+
+template <typename T, int EPI, int SP>
+int rows_launch_sp(const LinearArgs& a, hipStream_t st) {
+  constexpr int C = 16 / SP, KB = 4 * Vec16<T>::n;
+  const int row_tiles = (a.M + C - 1) / C, tiles = row_tiles * ((a.N + C - 1) / C);
+  const int nb = (a.K + KB - 1) / KB;
+  if (nb > 64)  // about one batch of loads per wave
+    rows_kernel<T, EPI, 16, SP><<<tiles, 1024, 0, st>>>(a, row_tiles, tiles);
+  else if (nb > 32)
+    rows_kernel<T, EPI, 8, SP><<<tiles, 512, 0, st>>>(a, row_tiles, tiles);
+  else
+    rows_kernel<T, EPI, 4, SP><<<tiles, 256, 0, st>>>(a, row_tiles, tiles);
+  NML_LAUNCHED();
+  return 0;
+}
+
+// As many column tiles as CUs, where the rows leave room for it.
+template <typename T, int EPI>
+int rows_launch(const LinearArgs& a, hipStream_t st) {
+  const int ct = (a.N + 15) / 16;
+  if (a.M <= 4 && ct < 128) return rows_launch_sp<T, EPI, 4>(a, st);
+  if (a.M <= 8 && ct < 256) return rows_launch_sp<T, EPI, 2>(a, st);
+  return rows_launch_sp<T, EPI, 1>(a, st);
 }
 
 // ------------------------------------------------------- skinny MFMA GEMM (fp16)
@@ -1368,12 +1497,8 @@ int linear_typed(const LinearArgs& a, hipStream_t st) {
     set_error("linear: fused RMSNorm needs the fp16 skinny path (8 < rows <= 64)");
     return -1;
   }
-  if (a.M <= 8) {
-    if (a.M <= 1) return gemv_dispatch_rpw<T, EPI, 1>(a, st);
-    if (a.M <= 2) return gemv_dispatch_rpw<T, EPI, 2>(a, st);
-    if (a.M <= 4) return gemv_dispatch_rpw<T, EPI, 4>(a, st);
-    return gemv_dispatch_rpw<T, EPI, 8>(a, st);
-  }
+  if (gemv_applies<T>(a)) return gemv_launch<T, EPI>(a, st);
+  if (rows_applies<T>(a)) return rows_launch<T, EPI>(a, st);
   if constexpr (sizeof(T) == 2) {
     if (big_gemm_applies(a)) return gemm_big_launch<EPI>(a, st);
   } else {
