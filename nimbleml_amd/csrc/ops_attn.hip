@@ -1152,6 +1152,9 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pipe_kernel(AttnArgs a) {
     if (j + 1 < nt) iter(I1{}, j + 1, sB, sA);
   }
   l += __shfl_xor(l, 32, 64);
+  if constexpr (kRounded) {
+    if (a.lse && myq < S && hi == 0) a.lse[static_cast<size_t>(bh) * a.S + myq] = m + logf(l);
+  }
   if (myq < S) {
     const float inv = 1.f / l;
     const int hd = a.H * dk;
@@ -1399,8 +1402,8 @@ int prefill_scalar(const AttnArgs& a, hipStream_t st) {
 }
 
 // Matrix cores where the call allows it. fp16 calls that keep the softmax statistics take
-// fp16-rounded scores, as the backward recomputes them: head dims 64 and 128 causal have such a
-// kernel. (The pipelined kernel's buffer loads take a 32-bit byte range per (row, head): a
+// fp16-rounded scores, as the backward recomputes them: the pipelined kernel where it rounds
+// them anyway, attn_prefill_mfma_kernel for head dims 64 and 128 causal. (The pipelined kernel's buffer loads take a 32-bit byte range per (row, head): a
 // cache row block past 2 GiB takes another kernel.)
 template <typename T>
 int prefill_matrix(const AttnArgs& a, hipStream_t st, bool* taken) {
@@ -1414,7 +1417,8 @@ int prefill_matrix(const AttnArgs& a, hipStream_t st, bool* taken) {
       }
     } else {
       const bool ranged = a.kv_stride_h * static_cast<long long>(sizeof(half_t)) < (1LL << 31);
-      if (!a.lse && !a.m_out && ranged) {
+      const bool rounded = mode == kMasked || (a.dk != 64 && a.dk != 128);
+      if ((!a.lse || rounded) && !a.m_out && ranged) {
         if (mode == kCausal) return prefill_pipe_mode<kCausal>(a, st);
         return mode == kFull ? prefill_pipe_mode<kFull>(a, st) : prefill_pipe_mode<kMasked>(a, st);
       }

@@ -1377,7 +1377,8 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_kernel(AttnBwdArgs a) {
   }
 }
 
-// ---- MFMA variant (head dims 64 and 128): 64 keys × 64 queries per step, 4 waves.
+// ---- MFMA variant (head dims up to 128, tiles padded to 32, 64, 96 or 128 columns; PAD: the
+// head dim is below DK): 64 keys × 64 queries per step, 4 waves.
 // Wave w = (wq, wk) = (w / 2, w % 2) takes the 32 × 32 sub-tile of queries 32·wq… and keys
 // 32·wk…; MFMA 32×32×2 fp32 throughout. A 32 × 32 result tile in registers holds, in
 // lane l and register r, row 8(r/4) + 4(l/32) + r%4 and column l%32; the products that
@@ -1407,26 +1408,26 @@ constexpr size_t attn_mfma_lds() {
   return (4 * kAT * (DK + 1) + 2 * kAT) * sizeof(float);
 }
 
-// rows [lo, lo + 64) of a head-major (S, DK) slice into a [64][DK + 1] tile (0 past S)
+// rows [lo, lo + 64) of a head-major (S, hd) slice into a [64][DK + 1] tile (0 past S and hd)
 template <int DK, typename T>
-__device__ __forceinline__ void tile_rows(float* dst, const T* __restrict__ src, int lo, int S) {
+__device__ __forceinline__ void tile_rows(float* dst, const T* __restrict__ src, int hd, int lo, int S) {
   for (int e = threadIdx.x; e < kAT * DK / 4; e += 256) {
     const int r = e / (DK / 4), c = (e - r * (DK / 4)) * 4;
     floatx4 v = {0.f, 0.f, 0.f, 0.f};
-    if (lo + r < S) v = ld4(src + static_cast<long long>(lo + r) * DK + c);
+    if (lo + r < S && c < hd) v = ld4(src + static_cast<long long>(lo + r) * hd + c);
 #pragma unroll
     for (int j = 0; j < 4; ++j) dst[r * (DK + 1) + c + j] = v[j];
   }
 }
 
-// rows [lo, lo + 64) of head h of a merged (B·S, H·DK) tensor
+// rows [lo, lo + 64) of head h of a merged (B·S, H·hd) tensor
 template <int DK, typename T>
-__device__ __forceinline__ void tile_merged(float* dst, const T* __restrict__ src, int b, int h,
+__device__ __forceinline__ void tile_merged(float* dst, const T* __restrict__ src, int hd, int b, int h,
                                             int H, int lo, int S) {
   for (int e = threadIdx.x; e < kAT * DK / 4; e += 256) {
     const int r = e / (DK / 4), c = (e - r * (DK / 4)) * 4;
     floatx4 v = {0.f, 0.f, 0.f, 0.f};
-    if (lo + r < S) v = ld4(src + (static_cast<long long>(b) * S + lo + r) * H * DK + h * DK + c);
+    if (lo + r < S && c < hd) v = ld4(src + (static_cast<long long>(b) * S + lo + r) * H * hd + h * hd + c);
 #pragma unroll
     for (int j = 0; j < 4; ++j) dst[r * (DK + 1) + c + j] = v[j];
   }
@@ -1439,14 +1440,14 @@ __device__ __forceinline__ int d_row(int r, int lane) { return 8 * (r >> 2) + 4 
 template <int DK, typename T>
 struct TileRegs {
   floatx4 v[DK / 16];
-  // rows [lo, lo + 64) of a row-major source with row stride ld (0 past S)
-  __device__ __forceinline__ void load(const T* __restrict__ src, long long ld, int lo, int S) {
+  // rows [lo, lo + 64) of a row-major source of hd columns, row stride ld (0 past S and hd)
+  __device__ __forceinline__ void load(const T* __restrict__ src, long long ld, int hd, int lo, int S) {
 #pragma unroll
     for (int i = 0; i < DK / 16; ++i) {
       const int e = threadIdx.x + 256 * i;
       const int r = e / (DK / 4), c = (e - r * (DK / 4)) * 4;
       const floatx4 z = {0.f, 0.f, 0.f, 0.f};
-      v[i] = lo + r < S ? ld4(src + static_cast<long long>(lo + r) * ld + c) : z;
+      v[i] = lo + r < S && c < hd ? ld4(src + static_cast<long long>(lo + r) * ld + c) : z;
     }
   }
   __device__ __forceinline__ void store(float* dst) const {
@@ -1461,10 +1462,11 @@ struct TileRegs {
 };
 
 // dK, dV of 64 keys; the query tiles from the key tile on.
-template <int DK, typename T>
+template <int DK, bool PAD, typename T>
 __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_mfma(AttnBwdArgs a) {
   extern __shared__ float lds[];
   constexpr int P = DK + 1, NJ = DK / 32;
+  const int hd = PAD ? a.dk : DK;
   float* Ks = lds;
   float* Vs = Ks + kAT * P;
   float* Qs = Vs + kAT * P;
@@ -1477,9 +1479,9 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_mfma(AttnBwdArgs a) {
   bwd_tile_order(bh, t);
   const int b = bh / a.H, h = bh - (bh / a.H) * a.H;
   const int S = a.S, k_lo = t * kAT;  // the longest key tiles (most query tiles) first
-  const long long hoff = static_cast<long long>(bh) * S * DK;
-  tile_rows<DK>(Ks, static_cast<const T*>(a.k) + hoff, k_lo, S);
-  tile_rows<DK>(Vs, static_cast<const T*>(a.v) + hoff, k_lo, S);
+  const long long hoff = static_cast<long long>(bh) * S * hd;
+  tile_rows<DK>(Ks, static_cast<const T*>(a.k) + hoff, hd, k_lo, S);
+  tile_rows<DK>(Vs, static_cast<const T*>(a.v) + hoff, hd, k_lo, S);
   floatx16 dv[NJ], dk[NJ];
 #pragma unroll
   for (int j = 0; j < NJ; ++j)
@@ -1487,13 +1489,13 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_mfma(AttnBwdArgs a) {
     for (int r = 0; r < 16; ++r) dv[j][r] = dk[j][r] = 0.f;
   const int key = k_lo + 32 * wk + l32;  // this lane's key (column of S)
   const float inv_scale = 1.0f / a.scale, mul = score_mul<T>(a.scale);
-  const T* dout_b = static_cast<const T*>(a.dout) + static_cast<long long>(b) * S * a.H * DK + h * DK;
+  const T* dout_b = static_cast<const T*>(a.dout) + static_cast<long long>(b) * S * a.H * hd + h * hd;
   const T* qg = static_cast<const T*>(a.q);
   TileRegs<DK, T> nq, no;
   float nl = 0.f, nd = 0.f;
   auto fetch = [&](int lo) {
-    nq.load(qg + hoff, DK, lo, S);
-    no.load(dout_b, static_cast<long long>(a.H) * DK, lo, S);
+    nq.load(qg + hoff, hd, hd, lo, S);
+    no.load(dout_b, static_cast<long long>(a.H) * hd, hd, lo, S);
     if (threadIdx.x < kAT) {
       const int q = lo + threadIdx.x;
       nl = q < S ? a.lse[static_cast<long long>(bh) * S + q] : 0.f;
@@ -1579,14 +1581,15 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_mfma(AttnBwdArgs a) {
   }
   __syncthreads();
   if (wq == 0) {
-    const int d = a.H * DK;
+    const int d = a.H * hd;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int kk = k_lo + 32 * wk + d_row(r, lane);
       if (kk < S) {
-        T* row = static_cast<T*>(a.dqkv) + (static_cast<long long>(b) * S + kk) * 3 * d + h * DK;
+        T* row = static_cast<T*>(a.dqkv) + (static_cast<long long>(b) * S + kk) * 3 * d + h * hd;
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
+          if (PAD && 32 * j + l32 >= hd) continue;
           row[d + 32 * j + l32] = static_cast<T>(dk[j][r] + red[(((wk * 2 + 1) * NJ + j) * 16 + r) * 64 + lane]);
           row[2 * d + 32 * j + l32] = static_cast<T>(dv[j][r] + red[(((wk * 2 + 0) * NJ + j) * 16 + r) * 64 + lane]);
         }
@@ -1597,10 +1600,11 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_mfma(AttnBwdArgs a) {
 
 // dQ of 64 queries; the key tiles up to the query tile. Wave w = (wk, wq) = (w / 2, w % 2)
 // computes Sᵀ (keys as rows) so that its registers feed dQ = dS·K as the A operand.
-template <int DK, typename T>
+template <int DK, bool PAD, typename T>
 __global__ __launch_bounds__(256) void attn_bwd_dq_mfma(AttnBwdArgs a) {
   extern __shared__ float lds[];
   constexpr int P = DK + 1, NJ = DK / 32;
+  const int hd = PAD ? a.dk : DK;
   float* Ks = lds;
   float* Vs = Ks + kAT * P;
   float* Qs = Vs + kAT * P;
@@ -1611,11 +1615,11 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_mfma(AttnBwdArgs a) {
   bwd_tile_order(bh, t);
   const int b = bh / a.H, h = bh - (bh / a.H) * a.H;
   const int S = a.S, q_lo = (gridDim.x - 1 - t) * kAT;  // the longest query tiles first
-  const long long hoff = static_cast<long long>(bh) * S * DK;
+  const long long hoff = static_cast<long long>(bh) * S * hd;
   const T* kg = static_cast<const T*>(a.k);
   const T* vg = static_cast<const T*>(a.v);
-  tile_rows<DK>(Qs, static_cast<const T*>(a.q) + hoff, q_lo, S);
-  tile_merged<DK>(Os, static_cast<const T*>(a.dout), b, h, a.H, q_lo, S);
+  tile_rows<DK>(Qs, static_cast<const T*>(a.q) + hoff, hd, q_lo, S);
+  tile_merged<DK>(Os, static_cast<const T*>(a.dout), hd, b, h, a.H, q_lo, S);
   const int q = q_lo + 32 * wq + l32;  // this lane's query (column of Sᵀ)
   const float lse = q < S ? a.lse[static_cast<long long>(bh) * S + q] : 0.f;
   const float dd = q < S ? a.dvec[static_cast<long long>(bh) * S + q] : 0.f;
@@ -1627,16 +1631,16 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_mfma(AttnBwdArgs a) {
   const int k_end = min(S, q_lo + kAT);
   const float inv_scale = 1.0f / a.scale, mul = score_mul<T>(a.scale);
   TileRegs<DK, T> nk, nv;
-  nk.load(kg + hoff, DK, 0, S);
-  nv.load(vg + hoff, DK, 0, S);
+  nk.load(kg + hoff, hd, hd, 0, S);
+  nv.load(vg + hoff, hd, hd, 0, S);
   for (int k_lo = 0; k_lo < k_end; k_lo += kAT) {
     __syncthreads();  // every wave is done with the previous tile
     nk.store(Ks);
     nv.store(Vs);
     __syncthreads();
     if (k_lo + kAT < k_end) {
-      nk.load(kg + hoff, DK, k_lo + kAT, S);
-      nv.load(vg + hoff, DK, k_lo + kAT, S);
+      nk.load(kg + hoff, hd, hd, k_lo + kAT, S);
+      nv.load(vg + hoff, hd, hd, k_lo + kAT, S);
     }
     floatx16 sc, dp;
 #pragma unroll
@@ -1677,15 +1681,15 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_mfma(AttnBwdArgs a) {
   }
   __syncthreads();
   if (wk == 0) {
-    const int d = a.H * DK;
+    const int d = a.H * hd;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int qq = q_lo + 32 * wq + d_row(r, lane);
       if (qq < S) {
-        T* row = static_cast<T*>(a.dqkv) + (static_cast<long long>(b) * S + qq) * 3 * d + h * DK;
+        T* row = static_cast<T*>(a.dqkv) + (static_cast<long long>(b) * S + qq) * 3 * d + h * hd;
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
-          row[32 * j + l32] = static_cast<T>(dq[j][r] + red[((wq * NJ + j) * 16 + r) * 64 + lane]);
+          if (!PAD || 32 * j + l32 < hd) row[32 * j + l32] = static_cast<T>(dq[j][r] + red[((wq * NJ + j) * 16 + r) * 64 + lane]);
       }
     }
   }
@@ -2089,36 +2093,54 @@ int attn_bwd_f16(const AttnBwdArgs& a, hipStream_t st) {
   return 0;
 }
 
-template <int DK, typename T>
+template <int DK, bool PAD, typename T>
 int attn_bwd_mfma(const AttnBwdArgs& a, hipStream_t st) {
   constexpr size_t lds = attn_mfma_lds<DK>();
   static bool attr = false;
   if (!attr) {
-    NML_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_bwd_dkdv_mfma<DK, T>),
+    NML_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_bwd_dkdv_mfma<DK, PAD, T>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-    NML_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_bwd_dq_mfma<DK, T>),
+    NML_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_bwd_dq_mfma<DK, PAD, T>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
     attr = true;
   }
   const dim3 grid((a.S + kAT - 1) / kAT, a.B * a.H);
-  attn_bwd_dkdv_mfma<DK, T><<<grid, 256, lds, st>>>(a);
+  attn_bwd_dkdv_mfma<DK, PAD, T><<<grid, 256, lds, st>>>(a);
   NML_LAUNCHED();
-  attn_bwd_dq_mfma<DK, T><<<grid, 256, lds, st>>>(a);
+  attn_bwd_dq_mfma<DK, PAD, T><<<grid, 256, lds, st>>>(a);
   NML_LAUNCHED();
   return 0;
 }
 
+// The matrix-core pair: causal, head dims up to 128 in 4-element pieces of aligned rows. fp16
+// head dims 64 and 128 on the fp16 MFMA, the rest widened to float32 as the scalar pair does.
+// (8 × 8 heads × 256 positions of 32 dims in float32: 94 + 75 µs on the scalar pair, 17 + 15
+// here.)
+template <typename T>
+bool attn_bwd_mfma_applies(const AttnBwdArgs& a) {
+  return !a.full && a.dk <= 128 && a.dk % 4 == 0 && !std::getenv("NIMBLEML_ATTN_BWD_VALU") &&
+         ((reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.k) |
+           reinterpret_cast<uintptr_t>(a.v) | reinterpret_cast<uintptr_t>(a.dout)) &
+          (4 * sizeof(T) - 1)) == 0;
+}
+
 template <int DK, typename T>
-int attn_bwd_dk(const AttnBwdArgs& a, hipStream_t st) {
-  if constexpr (DK == 64 || DK == 128) {
-    if (!a.full && !std::getenv("NIMBLEML_ATTN_BWD_VALU")) {  // MFMA kernels: causal only
-      if constexpr (sizeof(T) == 2) {
-        if (!std::getenv("NIMBLEML_TRAIN_F16_WIDEN")) return attn_bwd_f16<DK>(a, st);
-      }
-      return attn_bwd_mfma<DK, T>(a, st);
+int attn_bwd_mfma_dk(const AttnBwdArgs& a, hipStream_t st) {
+  return a.dk == DK ? attn_bwd_mfma<DK, false, T>(a, st) : attn_bwd_mfma<DK, true, T>(a, st);
+}
+
+template <typename T>
+int attn_bwd_matrix(const AttnBwdArgs& a, hipStream_t st) {
+  if constexpr (sizeof(T) == 2) {
+    if (!std::getenv("NIMBLEML_TRAIN_F16_WIDEN")) {
+      if (a.dk == 64) return attn_bwd_f16<64>(a, st);
+      if (a.dk == 128) return attn_bwd_f16<128>(a, st);
     }
   }
-  return attn_bwd_scalar<DK, T>(a, st);
+  if (a.dk <= 32) return attn_bwd_mfma_dk<32, T>(a, st);
+  if (a.dk <= 64) return attn_bwd_mfma_dk<64, T>(a, st);
+  if (a.dk <= 96) return attn_bwd_mfma_dk<96, T>(a, st);
+  return attn_bwd_mfma_dk<128, T>(a, st);
 }
 
 // --------------------------------------------------------------- RoPE backward
@@ -2395,14 +2417,10 @@ int attention_backward_t(const AttnBwdArgs& a, hipStream_t st) {
   const long long pairs = static_cast<long long>(a.B) * a.S * a.H;
   attn_bwd_dot_kernel<T><<<static_cast<int>((pairs + 3) / 4), 256, 0, st>>>(a);
   NML_LAUNCHED();
-  switch (a.dk) {
-    case 8: return attn_bwd_dk<8, T>(a, st);
-    case 16: return attn_bwd_dk<16, T>(a, st);
-    case 32: return attn_bwd_dk<32, T>(a, st);
-    case 64: return attn_bwd_dk<64, T>(a, st);
-    case 128: return attn_bwd_dk<128, T>(a, st);
-  }
-  // other head dims: the scalar kernels on tiles padded to 32, 64, 128 or 256 columns
+  if (attn_bwd_mfma_applies<T>(a)) return attn_bwd_matrix<T>(a, st);
+  if (a.dk == 8) return attn_bwd_scalar<8, T>(a, st);
+  if (a.dk == 16) return attn_bwd_scalar<16, T>(a, st);
+  // the scalar kernels, tiles padded to 32, 64, 128 or 256 columns
   if (a.dk < 1 || a.dk > kMaxHeadDim) {
     set_error("attention backward: head_dim %d outside [1, %d]", a.dk, kMaxHeadDim);
     return -1;
