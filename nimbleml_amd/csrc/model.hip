@@ -741,6 +741,7 @@ int nml_model_param_ptr(nml_model* m, int kind, int layer, void** ptr) {
   NML_REQUIRE(m != nullptr, "model is null");
   void** slot = param_slot(m, kind, layer);
   NML_REQUIRE(slot != nullptr, "unknown parameter kind %d / layer %d", kind, layer);
+  train_params_open(m);
   *ptr = *slot;
   return 0;
 }

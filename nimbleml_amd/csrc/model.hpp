@@ -85,6 +85,9 @@ int check_ready(nml_model* m);
 
 // Training state teardown (train.hip), called by nml_model_destroy.
 void train_release(nml_model* m);
+// Parameters change, or a caller gets a pointer to them: a backward of the last loss forms its
+// logits from the parameters that it finds.
+void train_params_open(nml_model* m);
 // After a parameter upload: an fp16 model's AdamW master copy of that parameter (when the
 // optimizer state exists) is taken again from the uploaded values.
 int train_param_uploaded(nml_model* m, const void* param, size_t elems);

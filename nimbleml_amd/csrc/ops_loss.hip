@@ -55,6 +55,84 @@ __global__ __launch_bounds__(256) void ce_rows_kernel(const T* __restrict__ logi
   }
 }
 
+// The same with the row in registers: one 16-byte read of every logit instead of two reads
+// element by element. V a multiple of the chunk's element count E, at most 256·NCH chunks,
+// rows 16-byte aligned; Σexp in another order. Bound by the exponentials (131 M of them, 4096
+// rows × 32000: fp16 252 → 94 µs, float32 277 → 110).
+template <typename T, int NCH>
+__global__ __launch_bounds__(256) void ce_rows_reg_kernel(const T* __restrict__ logits, int V,
+                                                          const int64_t* __restrict__ labels,
+                                                          long long ignore_index, int has_ignore,
+                                                          float* __restrict__ row_loss,
+                                                          int* __restrict__ row_valid,
+                                                          int* __restrict__ err) {
+#pragma clang fp contract(off)
+  constexpr int E = 16 / static_cast<int>(sizeof(T));
+  typedef T vec_t __attribute__((ext_vector_type(E)));
+  __shared__ float red[4];
+  const int row = blockIdx.x, tid = threadIdx.x, nch = V / E;
+  const T* l = logits + static_cast<size_t>(row) * V;
+  const int64_t y = labels[row];
+  const bool ignored = has_ignore && y == ignore_index;
+  if (ignored || y < 0 || y >= V) {
+    if (tid == 0) {
+      if (!ignored) atomicOr(err, 2);
+      row_loss[row] = 0.f;
+      row_valid[row] = 0;
+    }
+    return;
+  }
+  vec_t r[NCH];
+  float mx = -INFINITY;
+#pragma unroll
+  for (int k = 0; k < NCH; ++k) {  // (past the row: its last chunk again, summed by nobody)
+    const int c = min(tid + 256 * k, nch - 1);
+    r[k] = reinterpret_cast<const vec_t*>(l)[c];
+  }
+#pragma unroll
+  for (int k = 0; k < NCH; ++k)
+#pragma unroll
+    for (int e = 0; e < E; ++e) mx = fmaxf(mx, static_cast<float>(r[k][e]));
+  mx = wave_max(mx);
+  if ((tid & 63) == 0) red[tid >> 6] = mx;
+  __syncthreads();
+  mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  float s = 0.f;
+#pragma unroll
+  for (int k = 0; k < NCH; ++k)
+    if (tid + 256 * k < nch) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) s += rnd<T>(expf(rnd<T>(static_cast<float>(r[k][e]) - mx)));
+    }
+  s = block_sum(s, red);
+  if (tid == 0) {
+    const float lse = mx + logf(s);
+    row_loss[row] = lse - static_cast<float>(l[y]);
+    row_valid[row] = 1;
+  }
+}
+
+template <typename T>
+int ce_rows_launch(const T* l, int rows, int V, const int64_t* labels, long long ignore_index, int has_ignore,
+                   float* row_loss, int* row_valid, int* err, hipStream_t st) {
+  constexpr int E = 16 / static_cast<int>(sizeof(T));
+  const int per = (V / E + 255) / 256;
+  if (V % E == 0 && per <= 32 && (reinterpret_cast<uintptr_t>(l) & 15) == 0) {
+#define NML_CE_ROWS(NCHV)                                                                                \
+  ce_rows_reg_kernel<T, NCHV><<<rows, 256, 0, st>>>(l, V, labels, ignore_index, has_ignore, row_loss, row_valid, \
+                                                    err)
+    if (per <= 4) NML_CE_ROWS(4);
+    else if (per <= 8) NML_CE_ROWS(8);
+    else if (per <= 16) NML_CE_ROWS(16);
+    else NML_CE_ROWS(32);
+#undef NML_CE_ROWS
+  } else {
+    ce_rows_kernel<T><<<rows, 256, 0, st>>>(l, V, labels, ignore_index, has_ignore, row_loss, row_valid, err);
+  }
+  NML_LAUNCHED();
+  return 0;
+}
+
 // Rows of the fused head (EPI_CE partials), one wave per row: M = max of the tile maxima,
 // S = Σ_t s_t·exp(mx_t − M) (tiles in lane-strided order, then the wave sum), and the
 // row's loss lse − logit[label] with lse = M + log S, as ce_rows_kernel forms it.
@@ -144,13 +222,10 @@ int launch_ce_rows(int dt, const void* logits, int rows, int V, const int64_t* l
                    int* err, hipStream_t st) {
   if (rows == 0) return 0;
   if (dt == F16)
-    ce_rows_kernel<half_t><<<rows, 256, 0, st>>>((const half_t*)logits, V, labels, ignore_index,
-                                                 has_ignore, row_loss, row_valid, err);
-  else
-    ce_rows_kernel<float><<<rows, 256, 0, st>>>((const float*)logits, V, labels, ignore_index,
-                                                has_ignore, row_loss, row_valid, err);
-  NML_LAUNCHED();
-  return 0;
+    return ce_rows_launch(static_cast<const half_t*>(logits), rows, V, labels, ignore_index, has_ignore, row_loss,
+                          row_valid, err, st);
+  return ce_rows_launch(static_cast<const float*>(logits), rows, V, labels, ignore_index, has_ignore, row_loss,
+                        row_valid, err, st);
 }
 
 int launch_ce_combine(const float2* part, int tiles_n, const float* label_logit, int rows, int V,

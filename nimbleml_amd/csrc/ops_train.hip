@@ -1125,7 +1125,10 @@ __global__ __launch_bounds__(256) void ce_grad_reg_kernel(T* __restrict__ lg, in
   for (int k = 0; k < NCH; ++k)
     if (tid + 256 * k < nch) {
 #pragma unroll
-      for (int e = 0; e < E; ++e) se += rnd<T>(expf(rnd<T>(static_cast<float>(r[k][e]) - mx)));
+      for (int e = 0; e < E; ++e) {  // (the exponential, in T, takes the logit's place)
+        r[k][e] = static_cast<T>(expf(rnd<T>(static_cast<float>(r[k][e]) - mx)));
+        se += static_cast<float>(r[k][e]);
+      }
     }
   se = block_sum(se, red);
   const float inv = rnd<T>(1.0f / se);
@@ -1137,7 +1140,7 @@ __global__ __launch_bounds__(256) void ce_grad_reg_kernel(T* __restrict__ lg, in
       vec_t o;
 #pragma unroll
       for (int e = 0; e < E; ++e) {
-        float v = rnd<T>(rnd<T>(expf(rnd<T>(static_cast<float>(r[k][e]) - mx))) * inv);
+        float v = rnd<T>(static_cast<float>(r[k][e]) * inv);
         if (c * E + e == label) v = rnd<T>(v - 1.0f);
         o[e] = static_cast<T>(v * sc);
       }

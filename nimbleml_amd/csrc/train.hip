@@ -34,9 +34,11 @@ struct TrainState {
   Buf acts;     // saved activations of the last loss_train
   Buf scratch;  // backward scratch
   Buf io;       // ids and labels of the last loss_train, loss accumulators
+  Buf logits;   // the last loss_train's logits, where they were kept
   Buf mask;     // the (S, S) additive mask of a saved module forward, when it took one
   int B = 0, S = 0;
   bool saved = false;
+  bool logits_kept = false;  // `logits` holds them and no backward has used them up
   int what = 0;        // the saved forward: kSavedLoss, kSavedBlocks or kSavedMha
   int final_norm = 0;  // kSavedBlocks: the final RMSNorm ran after the blocks
   int full = 0;        // module forwards: non-causal attention
@@ -58,6 +60,7 @@ void train_release(nml_model* m) {
   m->train->masters.release();
   m->train->acts.release();
   m->train->scratch.release();
+  m->train->logits.release();
   m->train->io.release();
   delete m->train;
   m->train = nullptr;
@@ -123,6 +126,9 @@ int ensure_train(nml_model* m) {
   }
   return 0;
 }
+
+// Logits of a training forward kept for its backward: up to 4 GiB of the card's 288.
+constexpr size_t kKeptLogits = (size_t)4 << 30;
 
 // Rows per logits chunk: at most 512 MiB of logits at once.
 size_t logits_chunk(const nml_model* m, size_t R) {
@@ -387,7 +393,12 @@ MaskMode saved_mask(const TrainState* t) {
 
 }  // namespace
 
+void train_params_open(nml_model* m) {
+  if (m->train) m->train->logits_kept = false;
+}
+
 int train_param_uploaded(nml_model* m, const void* param, size_t elems) {
+  train_params_open(m);
   if (m->dt != F16 || !m->train || !m->train->masters.p) return 0;
   return launch_convert(F16, param, F32, static_cast<char*>(m->train->masters.p) + f32_off(m, param),
                         elems, nml::stream());
@@ -426,6 +437,7 @@ int nml_model_loss_train(nml_model* m, const int64_t* ids, const int64_t* labels
   NML_TRY(ensure_train(m));
   TrainState* t = m->train;
   t->saved = false;
+  t->logits_kept = false;
   const int B = (int)batch, S = (int)seq, R = B * S, d = m->d, dt = m->dt;
   const size_t es = m->es;
   if (R == 0) {
@@ -454,14 +466,21 @@ int nml_model_loss_train(nml_model* m, const int64_t* ids, const int64_t* labels
   NML_TRY(blocks_forward_saving(m, sv, B, S, MaskMode{}, st));
   NML_TRY(launch_rmsnorm(dt, sv.xl, m->lnf, sv.hf, nullptr, nullptr, R, d, kEps, st));
 
-  const size_t chunk = logits_chunk(m, R);
-  NML_TRY(m->logits_ws.ensure(align256(chunk * m->V * es)));
+  // The logits stay for the backward, which forms their gradient in place, where they are at
+  // most kKeptLogits bytes and there is room for them; else they are formed chunk by chunk,
+  // here and in the backward. (Forming them again cost a d 1024, V 32000, 4 × 1024 step 277 µs
+  // in fp16 and 1573 in float32.)
+  const size_t chunk = logits_chunk(m, R), all = (size_t)R * m->V * es;
+  const bool keep = all <= kKeptLogits && t->logits.ensure(align256(all)) == 0;
+  if (!keep) (void)hipGetLastError();  // no room is no error
+  if (!keep) NML_TRY(m->logits_ws.ensure(align256(chunk * m->V * es)));
   for (size_t r0 = 0; r0 < (size_t)R; r0 += chunk) {
     const int n = (int)(((size_t)R - r0 < chunk) ? (size_t)R - r0 : chunk);
-    NML_TRY(launch_linear(dt, lin(sv.hf + r0 * d * es, d, m->emb, nullptr, m->logits_ws.p, n, m->V,
-                                  d, EPI_NONE), st));
-    NML_TRY(launch_ce_rows(dt, m->logits_ws.p, n, m->V, dlab + r0, ignore_index, has_ignore,
-                           row_loss, row_valid, err, st));
+    void* lg = keep ? static_cast<char*>(t->logits.p) + r0 * m->V * es : m->logits_ws.p;
+    NML_TRY(launch_linear(dt, lin(sv.hf + r0 * d * es, d, m->emb, nullptr, lg, n, m->V, d, EPI_NONE),
+                          st));
+    NML_TRY(launch_ce_rows(dt, lg, n, m->V, dlab + r0, ignore_index, has_ignore, row_loss, row_valid,
+                           err, st));
     NML_TRY(launch_ce_reduce(row_loss, row_valid, n, acc, r0 > 0, st));
   }
   NML_TRY(launch_ce_finalize(acc, acc + 2, st));
@@ -479,6 +498,7 @@ int nml_model_loss_train(nml_model* m, const int64_t* ids, const int64_t* labels
   t->has_ignore = has_ignore;
   t->n_valid = host[1];
   t->what = kSavedLoss;
+  t->logits_kept = keep;
   t->saved = true;
   t->generation += 1;
   return 0;
@@ -510,12 +530,14 @@ int nml_model_backward(nml_model* m, double grad_scale) {
   // tied head + cross-entropy, chunk by chunk; dH lands in DX
   const float scale = static_cast<float>(grad_scale / t->n_valid);
   const size_t chunk = logits_chunk(m, R);
-  NML_TRY(m->logits_ws.ensure(align256(chunk * V * es)));
-  void* lg = m->logits_ws.p;
+  const bool kept = t->logits_kept;  // (a second backward of this loss forms them again)
+  t->logits_kept = false;
+  if (!kept) NML_TRY(m->logits_ws.ensure(align256(chunk * V * es)));
   for (size_t r0 = 0; r0 < (size_t)R; r0 += chunk) {
     const int n = (int)(((size_t)R - r0 < chunk) ? (size_t)R - r0 : chunk);
     const char* h = sv.hf + r0 * d * es;
-    NML_TRY(launch_linear(dt, lin(h, d, E, nullptr, lg, n, V, d, EPI_NONE), st));
+    void* lg = kept ? static_cast<char*>(t->logits.p) + r0 * V * es : m->logits_ws.p;
+    if (!kept) NML_TRY(launch_linear(dt, lin(h, d, E, nullptr, lg, n, V, d, EPI_NONE), st));
     NML_TRY(launch_ce_grad(dt, lg, n, V, dlab + r0, t->ignore_index, t->has_ignore, scale, st));
     NML_TRY(launch_gemm_bwd(dt, gb(lg, V, E, d, DX + r0 * d * es, d, n, d, V), true, false, GB_SET, st));
     NML_TRY(launch_gemm_bwd(dt, gb(lg, V, h, d, dE, d, V, d, n), false, false, GB_ADD, st));
@@ -699,6 +721,7 @@ int nml_model_adamw_step(nml_model* m, float lr, float beta1, float beta2, float
                          float bias_corr2, float eps, float weight_decay) {
   NML_TRY(check_ready(m));
   NML_TRY(ensure_adam(m));
+  train_params_open(m);
   TrainState* t = m->train;
   hipStream_t st = nml::stream();
   const size_t n_all = m->arena_bytes / m->es;

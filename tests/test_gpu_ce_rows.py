@@ -1,0 +1,74 @@
+"""The cross-entropy of logit rows held in registers: vocabularies at the edges of a thread's
+chunks and past them, ignored labels; and the training step whose backward uses the forward's
+logits and, the second time, forms them again."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from nimbleml_amd import _native as N
+from nimbleml_amd import kernels as K
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
+@pytest.mark.parametrize("vocab", [3, 8, 1023, 1024, 4096, 4104, 8200, 16392, 32768, 32776, 65544])
+def test_loss_over_vocab_edges(vocab, dtype):
+    r = np.random.RandomState(vocab)
+    h = r.randn(5, 64).astype(dtype)
+    w = (r.randn(vocab, 64) * 0.1).astype(dtype)
+    lab = r.randint(0, vocab, 5)
+    lab[3] = 1
+    x = h.astype(np.float64) @ w.astype(np.float64).T
+    lse = np.log(np.exp(x - x.max(-1, keepdims=True)).sum(-1)) + x.max(-1)
+    row = lse - x[np.arange(5), lab]
+    # fp16: the logits (below 4) and the shifted exponents rounded to 11 bits
+    tol = 4 * 2.0**-10 if dtype == np.float16 else 1e-5
+    assert abs(K.fused_tied_crossentropy_forward(h, w, lab) - row.mean()) <= tol
+    keep = lab != 1
+    if keep.any():
+        got = K.fused_tied_crossentropy_forward(h, w, lab, ignore_index=1)
+        assert abs(got - row[keep].mean()) <= tol
+
+
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
+def test_second_backward_of_a_loss_equals_the_first(dtype):
+    import nimbleml_amd as nm
+    from oracle.weights import TINY, make_weights, random_ids
+
+    cfg = TINY
+    w = make_weights(cfg, seed=3, dtype=dtype, rich=True)
+    m = nm.GPT.from_arrays(w, cfg.vocab_size, cfg.d_model, cfg.num_heads, cfg.num_layers,
+                           cfg.max_seq_len, dtype=dtype)
+    ids, lab = random_ids((2, 9), cfg.vocab_size, seed=5), random_ids((2, 9), cfg.vocab_size, seed=6)
+    h, loss = m._device_model(), C.c_double()
+    dids, dlab = N.DeviceArray.from_host(ids), N.DeviceArray.from_host(lab)
+    head = np.ascontiguousarray(w["token_emb.weights"])
+
+    def loss_train():
+        N.check(N.lib.nml_model_loss_train(h, dids.ptr, dlab.ptr, 2, 9, 0, 0, C.byref(loss)))
+
+    def set_head(scale):
+        arr = np.ascontiguousarray(head * np.asarray(scale, dtype))
+        N.check(N.lib.nml_model_set_param(h, N.P_TOKEN_EMB, 0, arr.ctypes.data, arr.nbytes))
+
+    def backward():
+        N.check(N.lib.nml_model_zero_grad(h))
+        N.check(N.lib.nml_model_backward(h, 1.0))
+        return [m._grad_array(k, 0, m._device_shape(k))
+                for k in (N.P_TOKEN_EMB, N.P_LN_F, N.P_WQKV, N.P_W1, N.P_B2)]
+
+    loss_train()
+    first, second = backward(), backward()
+    for x, y in zip(first, second):
+        assert np.abs(x).max() > 0 and np.array_equal(x, y)
+    # another head uploaded after the loss: its logits' gradient, in the first backward too
+    set_head(2)
+    changed = backward()
+    assert not np.array_equal(changed[0], first[0])
+    set_head(1)
+    loss_train()
+    set_head(2)
+    for x, y in zip(backward(), changed):
+        assert np.array_equal(x, y)
