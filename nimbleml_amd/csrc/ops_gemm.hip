@@ -375,6 +375,17 @@ __device__ __forceinline__ void epilogue_vec8(const LinearArgs& a, int m, int n,
     if (a.pre_out) *reinterpret_cast<half8*>(static_cast<half_t*>(a.pre_out) + row + n) = p;
 }
 
+// Runs of 8 columns are 16-byte accesses: rows and operands 16-byte aligned.
+template <int EPI>
+__device__ __forceinline__ bool run8_vec(const LinearArgs& a) {
+  uintptr_t ptrs = reinterpret_cast<uintptr_t>(a.out) | reinterpret_cast<uintptr_t>(a.bias) |
+                   reinterpret_cast<uintptr_t>(a.resid) | reinterpret_cast<uintptr_t>(a.pre_out);
+  if constexpr (EPI == EPI_QKV)
+    ptrs |= reinterpret_cast<uintptr_t>(a.qkv.q) | reinterpret_cast<uintptr_t>(a.qkv.k) |
+            reinterpret_cast<uintptr_t>(a.qkv.v);
+  return (a.N & 7) == 0 && (ptrs & 15) == 0;
+}
+
 template <int EPI, int TM, int TN>
 __device__ __forceinline__ void epilogue_staged(const LinearArgs& a, int m0, int n0,
                                                 const floatx16 (&acc)[TM / 64][TN / 128],
@@ -399,13 +410,7 @@ __device__ __forceinline__ void epilogue_staged(const LinearArgs& a, int m0, int
       }
   // (the wave reads back only its own region: its LDS operations complete in order)
   const int M = a.M, N = a.N;
-  uintptr_t ptrs = reinterpret_cast<uintptr_t>(a.out) | reinterpret_cast<uintptr_t>(a.bias) |
-                   reinterpret_cast<uintptr_t>(a.resid) | reinterpret_cast<uintptr_t>(a.pre_out);
-  if constexpr (EPI == EPI_QKV)
-    ptrs |= reinterpret_cast<uintptr_t>(a.qkv.q) | reinterpret_cast<uintptr_t>(a.qkv.k) |
-            reinterpret_cast<uintptr_t>(a.qkv.v);
-  const bool aligned = (ptrs & 15) == 0;
-  const bool vec8 = (N & 7) == 0 && aligned;
+  const bool vec8 = run8_vec<EPI>(a);
   constexpr int CH = C / 8;              // 16-byte runs per region row
   constexpr int IT = R * CH / 64;        // runs per lane
   // 256 × 256 GELU tiles: the tanh table sits right past the staging region
@@ -787,13 +792,151 @@ int gemm_big_launch(const LinearArgs& a, hipStream_t st) {
   return gemm_big_launch_gm<EPI, 4, kHM, kHN>(a, st);
 }
 
-// The direct-to-LDS kernels: K a multiple of 64, 16-byte aligned rows, and enough rows
+// The kernels on big::mainloop: K a multiple of 64, 16-byte aligned rows, and enough rows
 // for 128-row tiles to be mostly full.
 bool big_gemm_applies(const LinearArgs& a) {
   if (std::getenv("NIMBLEML_BIG_GEMM") && std::getenv("NIMBLEML_BIG_GEMM")[0] == '0') return false;
   if (a.K % kHK != 0 || a.lda % 8 != 0 || (reinterpret_cast<uintptr_t>(a.x) & 15) != 0) return false;
   if (big_gemm_wide(a)) return true;
   return a.M >= 256 && !(std::getenv("NIMBLEML_BIG_GEMM") && std::getenv("NIMBLEML_BIG_GEMM")[0] == 'w');
+}
+
+// ------------------------------------------------ fp16 GEMM of few tiles
+// An 8-wave workgroup owns a 64 × 64 output tile and divides K among its waves, so every byte
+// is read from LDS once. Stages of 128 k columns (64 x rows and 64 W rows: 32 KiB, each
+// 64-column half laid out as big::mainloop's) go through a ring of four by direct-to-LDS
+// loads: up to three are in flight while a fourth is multiplied. Wave w takes 16 columns of
+// each stage, MFMA 32×32×16 over the whole tile. The 8 partial tiles are summed through LDS in
+// a fixed order, 8 columns of a row per thread.
+// What bounds it: the bytes one CU pulls in with what it can have in flight (1 MB at K = 4096
+// in 13 µs), so more and smaller tiles on idle CUs beat fewer bytes in all. W2 and W_o of a
+// 512-row prompt (N = 1024: 32 tiles of 128 × 128, 128 of these) 39.7 → 16.8 µs at K = 4096,
+// 11.6 → 7.7 at K = 1024. Loads straight into fragments, without LDS: 31.7 and 11.0 (half
+// lines per load).
+struct T64 {
+  static constexpr int kRing = 4, kStage = 32 * 1024;
+  static constexpr int P = 64 + 4;  // floats per row of a partial tile: no bank conflicts
+  static constexpr size_t Lds = sizeof(float) * 8 * 64 * P;
+  static_assert(Lds >= static_cast<size_t>(kRing) * kStage, "the partial tiles take the ring's place");
+};
+
+template <int EPI>
+__global__ __launch_bounds__(512, 2) void gemm_f16_t64_kernel(LinearArgs a, int tiles_n, int tiles) {
+  extern __shared__ __attribute__((aligned(1024))) char lds_raw[];
+  float* part = reinterpret_cast<float*>(lds_raw);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = wave >> 2;
+  const int M = a.M, N = a.N, K = a.K, S = (K + 127) / 128;
+  int m0, n0;
+  big::tile_at<8>(big::xcd_tile(blockIdx.x, tiles), tiles_n, tiles, 64, 64, &m0, &n0);
+  // this wave's loads of a stage: blocks of 8 rows of its half, x rows (waves 0, 1, 4, 5) or
+  // W rows; rows past the last read the last, their products are not stored
+  const bool is_w = (wave & 2) != 0;
+  const half_t* src[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int row = 8 * ((wave & 1) * 4 + j) + (lane >> 3), ch = (lane & 7) ^ ((row >> 1) & 7);
+    src[j] = (is_w ? static_cast<const half_t*>(a.w) + static_cast<long long>(min(n0 + row, N - 1)) * K
+                   : static_cast<const half_t*>(a.x) + static_cast<long long>(min(m0 + row, M - 1)) * a.lda) +
+             ch * 8;
+  }
+  auto issue = [&](int s) {
+    // (a last stage of 64 columns: the second half's loads repeat the first's, unused)
+    const int kc = min(s * 128 + half * 64, K - 64);
+    char* dst = lds_raw + (s % T64::kRing) * T64::kStage + half * 16384 + (wave & 3) * 4096;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[j] + kc),
+                                       (__attribute__((address_space(3))) void*)(dst + j * 1024), 16, 0, 0);
+  };
+  floatx16 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds_raw)) + half * 16384;
+  const int fr = lane & 31, fc = 2 * (wave & 3) + (lane >> 5);
+  for (int s = 0; s < T64::kRing - 1 && s < S; ++s) issue(s);
+  for (int s = 0; s < S; ++s) {
+    // stage s has landed (4 loads per later stage may be outstanding), and every wave has read
+    // stage s − 1, whose buffer the new loads take
+    if (s + 2 < S)
+      asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+    else if (s + 1 < S)
+      asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    if (s + 3 < S) issue(s + 3);
+    const uint32_t base = lds0 + (s % T64::kRing) * T64::kStage;
+    half8 x0 = big::lds_read16(base + big::swz_off(fr, fc)), x1 = big::lds_read16(base + big::swz_off(32 + fr, fc));
+    half8 w0 = big::lds_read16(base + big::swz_off(64 + fr, fc)), w1 = big::lds_read16(base + big::swz_off(96 + fr, fc));
+    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(x0), "+v"(x1), "+v"(w0), "+v"(w1));
+    if (s * 128 + half * 64 < K) {
+      acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w0, x0, acc[0][0], 0, 0, 0);
+      acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w0, x1, acc[0][1], 0, 0, 0);
+      acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w1, x0, acc[1][0], 0, 0, 0);
+      acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w1, x1, acc[1][1], 0, 0, 0);
+    }
+  }
+  __syncthreads();
+  // D: lane l, register 4g + e → column 32i + 8g + 4(l/32) + e (W row) of row 32j + l%32
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        floatx4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = acc[i][j][4 * g + e];
+        *reinterpret_cast<floatx4*>(part + (wave * 64 + 32 * j + fr) * T64::P + 32 * i + 8 * g + 4 * (lane >> 5)) = v;
+      }
+  __syncthreads();
+  const int row = tid >> 3, c8 = (tid & 7) * 8, m = m0 + row, n = n0 + c8;
+  if (m >= M || n >= N) return;
+  floatx4 lo = {0.f, 0.f, 0.f, 0.f}, hi = lo;
+#pragma unroll
+  for (int w = 0; w < 8; ++w) {
+    const float* p = part + (w * 64 + row) * T64::P + c8;
+    lo += *reinterpret_cast<const floatx4*>(p);
+    hi += *reinterpret_cast<const floatx4*>(p + 4);
+  }
+  half8 o;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    o[e] = static_cast<half_t>(lo[e]);
+    o[4 + e] = static_cast<half_t>(hi[e]);
+  }
+  epilogue_run8<EPI>(a, m, n, o, run8_vec<EPI>(a) && n + 7 < N);
+}
+
+// One round of them, one per CU. Two rounds lose to 128 × 128 tiles (N 4096, K 1024: 384 rows
+// 13.7 against 12.3 µs, 512 rows 14.2 against 12.5) and beat gemm_f16_kernel below 256 rows
+// (17.2 whatever the tiles, and 55 at K 4096; 192 rows of N 1024: 7.6 and 16.3); at four,
+// N 32000, 128 rows, 27.8 against 23.4. K of at most 256 stays in the other kernels' order of
+// one chain (2 µs of launch and latency at stake).
+bool t64_applies(const LinearArgs& a) {
+  const char* e = std::getenv("NIMBLEML_BIG_GEMM");
+  if (e && (e[0] == '0' || e[0] == 'w')) return false;
+  const long long tiles = ((a.M + 63LL) / 64) * ((a.N + 63LL) / 64);
+  return a.K > 256 && a.K % 64 == 0 && tiles <= (a.M < 256 ? 512 : 256);
+}
+
+template <int EPI>
+int gemm_t64_launch(const LinearArgs& a, hipStream_t st) {
+  static bool attr = false;
+  if (!attr) {
+    NML_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f16_t64_kernel<EPI>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(T64::Lds)));
+    attr = true;
+  }
+  const int tiles_n = (a.N + 63) / 64, tiles = tiles_n * ((a.M + 63) / 64);
+  gemm_f16_t64_kernel<EPI><<<tiles, 512, T64::Lds, st>>>(a, tiles_n, tiles);
+  NML_LAUNCHED();
+  return 0;
 }
 
 // ------------------------------------------------ fp32 GEMM on the bf16 matrix cores
@@ -1500,6 +1643,7 @@ int linear_typed(const LinearArgs& a, hipStream_t st) {
   if (gemv_applies<T>(a)) return gemv_launch<T, EPI>(a, st);
   if (rows_applies<T>(a)) return rows_launch<T, EPI>(a, st);
   if constexpr (sizeof(T) == 2) {
+    if (t64_applies(a)) return gemm_t64_launch<EPI>(a, st);
     if (big_gemm_applies(a)) return gemm_big_launch<EPI>(a, st);
   } else {
     return gemm_f32_launch<EPI>(a, st);
