@@ -865,6 +865,8 @@ __global__ __launch_bounds__(kT) void decode_persist_kernel(PersistArgs a) {
       if (a.fuse_argmax) {
         a.tokens[pos + 1] = ii;
         a.pos[0] = pos + 1;
+      } else if (a.advance) {
+        a.pos[0] = pos + 1;
       }
       *a.epoch = ep + 1;
       NML_MARK(mh + 2);

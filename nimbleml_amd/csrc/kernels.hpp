@@ -141,6 +141,11 @@ struct AttnArgs {
   // (no pos_base, no ragged rows). Zero: causal.
   int full;
   const void* mask;
+  // Decode by length: sequence b has lens[b] keys, clamped into [1, lens_max] (a clamped
+  // length sets bit 0 of *lens_err where that is non-null), and `pos` is not read. Null: pos.
+  const int32_t* lens;
+  int lens_max;
+  int* lens_err;
 };
 int launch_attention_prefill(int dt, const AttnArgs& a, hipStream_t st);
 
@@ -285,13 +290,14 @@ struct PersistArgs {
   void* vc;
   long long kv_layer, kv_head; // elements between layers / heads
   int64_t* tokens;             // token history of the row; tokens[pos] is fed
-  int32_t* pos;                // pos[0]: position of the fed token (advanced when fused)
+  int32_t* pos;                // pos[0]: position of the fed token
   void* logits;                // (V) logits of the step
   unsigned long long* slots;   // exchange slots, persist_slot_count() entries, zeroed
   uint32_t* epoch;             // step counter, ≥ 1, advanced by the kernel
   int* err;                    // bit 0: token/position out of range; bit 2: exchange timeout
   int V, L, P;
   int fuse_argmax;             // greedy: write tokens[pos+1] and advance pos in-kernel
+  int advance;                 // without fuse_argmax: advance pos in-kernel all the same
   float scale;                 // sqrt(dk)
   // Optional phase timestamps (wall_clock64) of each workgroup: trace[g·stride + mark],
   // stride = persist_trace_stride(L), and at mark 2 the workgroup's XCD. Null: no tracing.

