@@ -849,9 +849,11 @@ __global__ __launch_bounds__(kT) void decode_persist_kernel(PersistArgs a) {
         i = oi;
       }
     }
+    // (advance: −1 where a wait gave up, so that pos stays while a workgroup may not have read it)
+    const bool lost = a.advance && __any(bad);
     if (lane == 0) {
       s_red[wave] = b;
-      s_redi[wave] = i;
+      s_redi[wave] = lost ? -1 : i;
     }
     __syncthreads();
     if (tid == 0) {
@@ -865,7 +867,7 @@ __global__ __launch_bounds__(kT) void decode_persist_kernel(PersistArgs a) {
       if (a.fuse_argmax) {
         a.tokens[pos + 1] = ii;
         a.pos[0] = pos + 1;
-      } else if (a.advance) {
+      } else if (a.advance && min(min(s_redi[0], s_redi[1]), min(s_redi[2], s_redi[3])) >= 0) {
         a.pos[0] = pos + 1;
       }
       *a.epoch = ep + 1;

@@ -1411,8 +1411,9 @@ int prefill_scalar(const AttnArgs& a, hipStream_t st) {
 
 // Matrix cores where the call allows it. fp16 calls that keep the softmax statistics take
 // fp16-rounded scores, as the backward recomputes them: the pipelined kernel where it rounds
-// them anyway, attn_prefill_mfma_kernel for head dims 64 and 128 causal. (The pipelined kernel's buffer loads take a 32-bit byte range per (row, head): a
-// cache row block past 2 GiB takes another kernel.)
+// them anyway, attn_prefill_mfma_kernel for head dims 64 and 128 causal. (The pipelined
+// kernel's buffer loads take a 32-bit byte range per (row, head): a cache row block past 2 GiB
+// takes another kernel.)
 template <typename T>
 int prefill_matrix(const AttnArgs& a, hipStream_t st, bool* taken) {
   *taken = true;

@@ -1040,12 +1040,14 @@ __global__ __launch_bounds__(256) void gemv_kernel(LinearArgs a) {
     }
 }
 
-// One row; up to 8 of at most 256 values, which one trip of a wave holds (K 256, 8 rows: 4.9 µs
-// here, 5.3 in rows_kernel); two float32 rows against a tied head (N 32000: 28.8 µs here,
-// 30.1 there; at 4 rows 34.0 against 33.1).
+// One row; up to 8 fp16 ones of at most 256 values, which one trip of a wave holds (K 256, 8
+// rows: 4.9 µs here, 5.3 in rows_kernel); up to 8 float32 rows: the 64 short chains of a wave
+// keep the sum closer to the exact one than the matrix cores' longer ones (K 1088, 8 rows:
+// relative error 0.9e-7 here, 1.5e-7 in rows_kernel, which took 11.8 µs for the 28.5 here at
+// K 4096, N 1024).
 template <typename T>
 bool gemv_applies(const LinearArgs& a) {
-  return a.M == 1 || (a.M <= 8 && a.K <= 256) || (sizeof(T) == 4 && a.M == 2 && a.N >= 8192);
+  return a.M == 1 || (a.M <= 8 && (sizeof(T) == 4 || a.K <= 256));
 }
 
 template <typename T, int EPI, int MR>
@@ -1079,10 +1081,10 @@ int gemv_launch(const LinearArgs& a, hipStream_t st) {
 // XCD, whose L2 holds their W rows.
 // What bounds it: one round trip of the loads and, at float32 with many rows, x's rows from
 // L2 (every column tile reads all of them). SP is for narrow outputs: N = 1024 is 64
-// workgroups of 16 columns, too few to pull 16 MB of W at K = 4096 (8 float32 rows: 17.8 µs
+// workgroups of 16 columns, too few to pull W at K = 4096 (measured on 16 MB of it: 17.8 µs
 // with SP 1, 11.8 with 2).
 // It replaces a GEMV of one wave per output (one round trip per 512 k: K 4096, N 1024, 8
-// rows 13.5 → 6.3 µs fp16, 28.5 → 11.8 float32) and 128 × 128 GEMM tiles on a few CUs (48
+// fp16 rows 13.5 → 6.3 µs) and 128 × 128 GEMM tiles on a few CUs (48
 // float32 rows: 302 → 20 µs).
 template <typename T, int EPI, int NW, int SP>
 __global__ __launch_bounds__(64 * NW) void rows_kernel(LinearArgs a, int row_tiles, int tiles) {
@@ -1145,8 +1147,8 @@ __global__ __launch_bounds__(64 * NW) void rows_kernel(LinearArgs a, int row_til
 }
 
 // fp16: 2 … 8 rows (the skinny kernel takes 9 … 64 where K is a multiple of 128, this one the
-// others of more than 256). float32: up to 16 rows, and more while the output is at most 1024 tiles of 16 × 16:
-// a round of 256 tiles costs 4.8 µs per 1024 of K, the 64 × 64 tile kernel about 20 however
+// others of more than 256). float32: 9 to 16 rows, and more while the output is at most 1024
+// tiles of 16 × 16: a round of 256 tiles costs 4.8 µs per 1024 of K, the 64 × 64 tile kernel about 20 however
 // few tiles it has (N 4096, K 1024: 64 rows 19.2 µs, 96 rows 26.7 against 21.1; N 1024: 256
 // rows 18.1 against 20.4, 384 rows 25.6 against 20.8; N 32000: 16 rows 41 against 55, 32 rows
 // 70 against 55).
@@ -1176,8 +1178,10 @@ int rows_launch_sp(const LinearArgs& a, hipStream_t st) {
 template <typename T, int EPI>
 int rows_launch(const LinearArgs& a, hipStream_t st) {
   const int ct = (a.N + 15) / 16;
-  if (a.M <= 4 && ct < 128) return rows_launch_sp<T, EPI, 4>(a, st);
-  if (a.M <= 8 && ct < 256) return rows_launch_sp<T, EPI, 2>(a, st);
+  if constexpr (sizeof(T) == 2) {  // (float32 has more rows)
+    if (a.M <= 4 && ct < 128) return rows_launch_sp<T, EPI, 4>(a, st);
+    if (a.M <= 8 && ct < 256) return rows_launch_sp<T, EPI, 2>(a, st);
+  }
   return rows_launch_sp<T, EPI, 1>(a, st);
 }
 
