@@ -1163,8 +1163,70 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pipe_kernel(AttnArgs a) {
   if constexpr (kRounded) {
     if (a.lse && myq < S && hi == 0) a.lse[static_cast<size_t>(bh) * a.S + myq] = m + logf(l);
   }
+  const float inv = 1.f / l;
+#pragma unroll
+  for (int ot = 0; ot < OT; ++ot)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[ot][r] *= inv;
+  if constexpr (EXACT) {
+    // An infinite or NaN value makes 0·∞ or ∞ − ∞ of keys that have no weight and of a
+    // probability's second part: outputs that are not finite though the softmax is are formed
+    // again key by key in float32, keys without weight left out (see the scalar kernel).
+    bool bad = false;
+#pragma unroll
+    for (int ot = 0; ot < OT; ++ot)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) bad |= !__builtin_isfinite(o[ot][r]);
+    bad = bad && myq < S && l > 0.f && __builtin_isfinite(l) && __builtin_isfinite(m);
+    if (__any(bad)) {
+      const int last = MODE == kCausal ? qpos : kend - 1;
+      const int jend = min(kend, ntw * kFK);
+      floatx16 w[OT];
+      float lw = 0.f;
+#pragma unroll
+      for (int ot = 0; ot < OT; ++ot)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) w[ot][r] = 0.f;
+      for (int j = 0; j < jend; ++j) {
+        const half_t* kr = Kg + static_cast<long long>(j) * dk + hi * 8;
+        const half_t* vr = Vg + static_cast<long long>(j) * dk + 4 * hi;
+        float s = 0.f;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+          if (!PAD || ks * 16 + hi * 8 < dk) {
+            const half8 kk = *reinterpret_cast<const half8*>(kr + ks * 16);
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+              s = __builtin_fmaf(static_cast<float>(qb[ks][e]), static_cast<float>(kk[e]), s);
+          }
+        s += __shfl_xor(s, 32, 64);
+        if constexpr (kRounded) {
+          half_t v = round_score(s);
+          if constexpr (MODE == kMasked) v = v + mrow[j];
+          s = static_cast<float>(v);
+        }
+        const float p = j > last ? 0.f : __builtin_amdgcn_exp2f((s - m) * cscale);
+        lw += p;
+#pragma unroll
+        for (int ot = 0; ot < OT; ++ot)
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+            if (p != 0.f && (!PAD || ot * 32 + 8 * g + 4 * hi < dk)) {
+              const half4 vv = *reinterpret_cast<const half4*>(vr + ot * 32 + 8 * g);
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                w[ot][4 * g + e] = __builtin_fmaf(p, static_cast<float>(vv[e]), w[ot][4 * g + e]);
+            }
+      }
+      const float winv = 1.f / lw;
+#pragma unroll
+      for (int ot = 0; ot < OT; ++ot)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (bad && !__builtin_isfinite(o[ot][r])) o[ot][r] = w[ot][r] * winv;
+    }
+  }
   if (myq < S) {
-    const float inv = 1.f / l;
     const int hd = a.H * dk;
     const size_t row = (a.row_start ? a.row_start[b] : static_cast<size_t>(b) * S) + myq;
     half_t* out = static_cast<half_t*>(a.out) + row * hd + h * dk;
@@ -1173,7 +1235,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pipe_kernel(AttnArgs a) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int d = ot * 32 + 8 * (r >> 2) + 4 * hi + (r & 3);
-        if (!PAD || d < dk) out[d] = static_cast<half_t>(o[ot][r] * inv);
+        if (!PAD || d < dk) out[d] = static_cast<half_t>(o[ot][r]);
       }
   }
 }
@@ -1316,16 +1378,64 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_mfma(AttnArgs a) {
           o[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(vrow[32 * j], sc[t][r], o[j], 0, 0, 0);
       }
   }
+  const float inv = 1.f / l;
+#pragma unroll
+  for (int j = 0; j < NJ; ++j)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[j][r] *= inv;
+  if constexpr (MODE != kCausal || PAD || (DK != 64 && DK != 128)) {
+    // as in attn_prefill_pipe_kernel: an infinite or NaN value of a key without weight
+    bool bad = false;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) bad |= !__builtin_isfinite(o[j][r]);
+    bad = bad && valid && l > 0.f && __builtin_isfinite(l) && __builtin_isfinite(m);
+    if (__any(bad)) {
+      floatx16 wo[NJ];
+      float lw = 0.f;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) wo[j][r] = 0.f;
+      for (int key = 0; key <= wave_last; ++key) {
+        const float* kr = K + static_cast<long long>(key) * dk + hi;
+        const float* vr = V + static_cast<long long>(key) * dk + 4 * hi;
+        float x = 0.f;
+#pragma unroll
+        for (int i = 0; i < DK / 2; ++i)
+          if (!PAD || 2 * i + hi < dk) x = __builtin_fmaf(qr[i], kr[2 * i], x);
+        x = (x + __shfl_xor(x, 32, 64)) / a.scale;
+        if constexpr (MODE == kMasked) x += mrow[key];
+        const float p = key > last ? 0.f : expf(x - m);
+        lw += p;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+            if (p != 0.f && (!PAD || 32 * j + 8 * g + 4 * hi < dk)) {
+              const floatx4 vv = *reinterpret_cast<const floatx4*>(vr + 32 * j + 8 * g);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) wo[j][4 * g + e] = __builtin_fmaf(p, vv[e], wo[j][4 * g + e]);
+            }
+      }
+      const float winv = 1.f / lw;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (bad && !__builtin_isfinite(o[j][r])) o[j][r] = wo[j][r] * winv;
+    }
+  }
   if (valid) {
     const size_t row = (a.row_start ? a.row_start[b] : static_cast<size_t>(b) * a.S) + s;
     float* out = static_cast<float*>(a.out) + row * a.H * dk + h * dk;
-    const float inv = 1.f / l;
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int d = 32 * j + 8 * (r >> 2) + 4 * hi + (r & 3);
-        if (!PAD || d < dk) out[d] = o[j][r] * inv;
+        if (!PAD || d < dk) out[d] = o[j][r];
       }
     if (a.lse && hi == 0) a.lse[static_cast<size_t>(bh) * a.S + s] = m + logf(l);
     if (a.m_out && hi == 0) {

@@ -99,3 +99,37 @@ def test_misaligned_rows_take_the_scalar_kernels(dtype):
                                           8.0, 0, N.np_dtype_code(dtype)))
     want = reference(q, k, v, None)
     assert np.abs(out.numpy() - want).max() <= TOL[dtype] * np.abs(v).max()
+
+
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
+@pytest.mark.parametrize("mode", ["full", "causal", "window", "bias", "causal call"])
+@pytest.mark.parametrize("seq,dk", [(90, 32), (200, 64), (130, 48), (150, 96), (70, 104), (150, 128)])
+def test_infinite_and_nan_values(seq, dk, mode, dtype):
+    """An infinite value is an infinite output wherever its key has a weight, and no output where
+    it has none (a masked key, or a later key of the same tile)."""
+    from nimbleml_amd import _native as N
+
+    if mode.startswith("causal") and dk in (64, 128):
+        pytest.skip("the causal kernel of these head dims sums every key of a tile, weight or not")
+    q, k, v = inputs(2, seq, dk, dtype)
+    v[0, 66, 1], v[0, 40, dk - 1] = np.inf, -np.inf
+    v[1, 3, 2], v[1, 60, 0], v[1, 61, 0] = np.nan, np.inf, -np.inf
+    bias = np.triu(np.full((seq, seq), -np.inf, dtype), 1) if mode == "causal call" else bias_of(mode, seq, dtype)
+    dev = [N.DeviceArray.from_host(a) for a in (q, k, v)]
+    if mode == "causal call":
+        out = N.DeviceArray((2, seq, dk), dtype)
+        N.check(N.lib.nml_sdpa_forward_device(*(d.ptr for d in dev), None, out.ptr, 2, seq, dk,
+                                              float(np.sqrt(dk)), 1, N.np_dtype_code(dtype)))
+        got = out.numpy()
+    else:
+        got = K.fused_sdpa_forward(q, k, v, np.sqrt(dk), bias)[0].numpy()
+    seen = np.ones((seq, seq), bool) if bias is None else np.isfinite(bias)
+    want = reference(q, k, np.where(np.isfinite(v), v, 0), bias)
+    for b, key, d, value in [(0, 66, 1, np.inf), (0, 40, dk - 1, -np.inf), (1, 3, 2, np.nan), (1, 60, 0, np.inf),
+                             (1, 61, 0, -np.inf)]:
+        with np.errstate(invalid="ignore"):  # inf - inf
+            want[b, :, d] = np.where(seen[:, key], want[b, :, d] + value, want[b, :, d])
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)].astype(dtype))
+    keep = np.isfinite(want)
+    assert np.abs(got[keep] - want[keep]).max() <= TOL[dtype] * 5  # |v| below 5
