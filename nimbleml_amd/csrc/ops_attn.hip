@@ -802,7 +802,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_kernel(AttnArgs a) {
 //      buffers each: K(j + 2) replaces K(j), read one iteration earlier; V(j + 1)
 //      replaces V(j − 1)), and the loads of K(j + 3) and V(j + 2) are issued;
 //   2. the rescale of O and l when tile j moved a query's reference point (rare: the
-//      point moves only when a maximum grows by more than 2^8 in p);
+//      point moves only when a maximum grows by more than 2^8 in p, 2^3 with EXACT);
 //   3. the scores of tile j + 1 (16 MFMAs) beside the probabilities of tile j (exp2,
 //      fp16 packing, row sums) — independent work for the matrix and vector pipes;
 //   4. P·V of tile j (16 MFMAs) beside the masking, maximum and reference point of
@@ -812,9 +812,12 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_kernel(AttnArgs a) {
 // past the sequence skip the arithmetic but join the barriers.
 //
 // MODE: causal; full (every key); or full with an additive (S, S) mask. PAD: the head dim
-// a.dk (a multiple of 8) is below DK: dims past it read as zero and are not stored. EXACT: the
-// probabilities enter P·V as two fp16 parts (22 bits) and two products, which leaves them the
-// float32 precision of the scalar kernels (every call but causal head dims 64 and 128). The
+// a.dk (a multiple of 8) is below DK: dims past it read as zero and are not stored. EXACT (every
+// call but causal head dims 64 and 128): the probabilities, times kUp = 2^12, enter P·V as two
+// fp16 parts and two products. Relative to the reference point's 1, p is then off by at most
+// 2^-24·p or, below 2^-13 where the second part leaves fp16's normal range, 2^-37: less than
+// half an ulp of a float32 sum over 2^13 such keys. (The reference point follows a maximum that
+// grew by more than 2^3, so that 2^12·p stays below fp16's 65504.) The
 // scores stay float32 accumulators at head dims 64 and 128; at others, and masked, they are
 // rounded as the reference's fp16 ops round them, rnd(rnd(rnd(q·k) / scale) + mask): a mask of
 // the type's lowest value must absorb the score, and the logits of small models are held
@@ -859,7 +862,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pipe_kernel(AttnArgs a) {
   // the scores' unit: q·k, or the rounded (and masked) score
   constexpr bool kRounded = MODE == kMasked || PAD || (DK != 64 && DK != 128);
   const float cscale = kRounded ? 1.4426950408889634f : 1.4426950408889634f / scale_t;
-  const float lazy = 8.0f / cscale;  // 2^8 in p
+  constexpr float kUp = EXACT ? 4096.f : 1.f;        // factor of every p (and so of l and o)
+  const float lazy = (EXACT ? 3.0f : 8.0f) / cscale;  // the growth left alone: 2^3 or 2^8 in p
   const int qw = q0 + wave * 32;     // first query of this wave
   const int myq = qw + (lane & 31);  // this lane's query
   const int hi = lane >> 5;          // which half of the wave
@@ -1045,8 +1049,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pipe_kernel(AttnArgs a) {
     constexpr int PAR = decltype(par_c)::value;
     constexpr bool NEXT = decltype(next_c)::value;
     if (grow) {
-      float alpha = __builtin_amdgcn_exp2f((m - mnew) * cscale);
-      if (MODE == kMasked && mnew == -INFINITY) alpha = 1.f;  // nothing summed yet
+      float alpha = __builtin_amdgcn_exp2f(MODE == kMasked ? (m - mnew) * cscale : m * cscale - mnew * cscale);
+      if (kRounded && mnew == -INFINITY) alpha = 1.f;  // nothing summed yet
       l *= alpha;
 #pragma unroll
       for (int t = 0; t < OT; ++t)
@@ -1060,9 +1064,10 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pipe_kernel(AttnArgs a) {
     if constexpr (kPin) __builtin_amdgcn_sched_barrier(0);
     if constexpr (NEXT) scores(std::integral_constant<int, PAR ^ 1>{}, nxt);
     if constexpr (kPin) __builtin_amdgcn_sched_barrier(0);
-    const float nmx = -m * cscale;
-    // (a masked score may be of the type's lowest value: the difference is formed first)
-    const float mref = MODE == kMasked && m == -INFINITY ? 0.f : m;
+    // (a masked score may be of the type's lowest value: the difference is formed first; else
+    // the reference point is the rounded m·cscale itself)
+    const float mref = kRounded && m == -INFINITY ? 0.f : m;
+    const float nmx = -mref * cscale;
     auto prob = [&](float s) {
       if constexpr (MODE == kMasked)
         return __builtin_amdgcn_exp2f((s - mref) * cscale);
@@ -1076,13 +1081,13 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pipe_kernel(AttnArgs a) {
       for (int jj = 0; jj < 8; jj += 2) {
         const float p0 = prob(cur[blk >> 1][8 * (blk & 1) + jj]);
         const float p1 = prob(cur[blk >> 1][8 * (blk & 1) + jj + 1]);
-        const half2v pp = {static_cast<_Float16>(p0), static_cast<_Float16>(p1)};
+        const half2v pp = {static_cast<_Float16>(p0 * kUp), static_cast<_Float16>(p1 * kUp)};
         l = __builtin_amdgcn_fdot2(pp, ones, l, false);
         pb[blk][jj] = pp[0];
         pb[blk][jj + 1] = pp[1];
-        if constexpr (EXACT) {
-          const half2v pr = {static_cast<_Float16>(p0 - static_cast<float>(pp[0])),
-                             static_cast<_Float16>(p1 - static_cast<float>(pp[1]))};
+        if constexpr (EXACT) {  // (fma: one mixed-precision instruction a part)
+          const half2v pr = {static_cast<_Float16>(__builtin_fmaf(p0, kUp, -static_cast<float>(pp[0]))),
+                             static_cast<_Float16>(__builtin_fmaf(p1, kUp, -static_cast<float>(pp[1])))};
           l = __builtin_amdgcn_fdot2(pr, ones, l, false);
           pl[blk][jj] = pr[0];
           pl[blk][jj + 1] = pr[1];
@@ -1161,7 +1166,13 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pipe_kernel(AttnArgs a) {
   }
   l += __shfl_xor(l, 32, 64);
   if constexpr (kRounded) {
-    if (a.lse && myq < S && hi == 0) a.lse[static_cast<size_t>(bh) * a.S + myq] = m + logf(l);
+    // (ln 2 in two parts: the reference point of unmasked scores is m·cscale as rounded)
+    if (a.lse && myq < S && hi == 0) {
+      const float m2 = m * cscale, ll = logf(l * (1.f / kUp));
+      a.lse[static_cast<size_t>(bh) * a.S + myq] =
+          MODE == kMasked ? m + ll
+                          : __builtin_fmaf(m2, 0.693147182f, __builtin_fmaf(m2, -1.90465430e-9f, ll));
+    }
   }
   const float inv = 1.f / l;
 #pragma unroll

@@ -133,3 +133,25 @@ def test_infinite_and_nan_values(seq, dk, mode, dtype):
     assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)].astype(dtype))
     keep = np.isfinite(want)
     assert np.abs(got[keep] - want[keep]).max() <= TOL[dtype] * 5  # |v| below 5
+
+
+@pytest.mark.parametrize("gap", [6.0, 11.0, 15.0, 18.0])
+@pytest.mark.parametrize("mode", ["full", "bias"])
+@pytest.mark.parametrize("dk", [32, 64, 96, 128])
+def test_many_small_probabilities_beside_a_peak(dk, mode, gap):
+    """One key above thousands of equal ones, whose weight times their values is the result: each
+    probability is off by at most 2^-24 of itself or 2^-37 of the peak's."""
+    seq, value = 3000, 30000.0
+    q, k, v = (np.zeros((1, seq, dk), np.float16) for _ in range(3))
+    q[..., 0], v[:] = 1, value
+    bias = np.zeros((seq, seq), np.float16) if mode == "bias" else None
+    v[0, 1717] = 0
+    if bias is None:
+        k[0, 1717, 0] = gap
+    else:
+        bias[:, 1717] = gap
+    got = K.fused_sdpa_forward(q, k, v, 1.0, bias)[0].numpy()
+    p = (seq - 1) * np.exp(-gap)
+    want = value * p / (1 + p)
+    # the output's rounding (2^-11), a float32 sum of `seq` terms, and the bound above
+    assert np.abs(got - want).max() <= want * (2.0**-11 + seq * 2.0**-24) + seq * value * 2.0**-37
