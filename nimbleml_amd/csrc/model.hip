@@ -1012,7 +1012,13 @@ int nml_model_forward_cached(nml_model* m, nml_cache* c, const int64_t* ids, siz
     NML_HIP(hipMemcpyAsync(&herr, c->err, sizeof(int), hipMemcpyDeviceToHost, st));
     NML_HIP(hipStreamSynchronize(st));
     m->last_decode_persistent = 1;
-    if (herr & 4) c->len[0] -= 1;  // the step did not advance its position
+    if (herr & 4) {
+      // The step is not taken. Whether the device advanced its position depends on which
+      // workgroup gave up, so both sides are set.
+      c->len[0] -= 1;
+      NML_HIP(hipMemcpyAsync(c->len_dev, c->len.data(), sizeof(int32_t), hipMemcpyHostToDevice, st));
+      NML_HIP(hipStreamSynchronize(st));
+    }
     NML_REQUIRE((herr & 4) == 0, "persistent decode: a data exchange timed out");
     NML_REQUIRE(herr == 0, "Token ID out of range [0, %d)", m->V);
     return 0;
