@@ -777,7 +777,8 @@ int nml_model_param_ptr(nml_model* m, int kind, int layer, void** ptr) {
   NML_REQUIRE(m != nullptr, "model is null");
   void** slot = param_slot(m, kind, layer);
   NML_REQUIRE(slot != nullptr, "unknown parameter kind %d / layer %d", kind, layer);
-  train_params_open(m);
+  if (!m->params_out) train_params_open(m);
+  m->params_out = true;
   *ptr = *slot;
   return 0;
 }

@@ -62,6 +62,7 @@ struct nml_model {
   nml::Buf small;      // device counters, positions, loss accumulators
   nml::Buf persist;    // persistent decode: layer pointer table, exchange slots, epoch
   nml::Buf ragged;     // packed ragged prefill: row table, lengths, row starts
+  bool params_out = false;           // a caller holds pointers into the parameters
   nml::TrainState* train = nullptr;  // gradients and saved activations, once enabled
   // decode timing of the last generate()
   float last_decode_ms = 0.f;
@@ -85,8 +86,8 @@ int check_ready(nml_model* m);
 
 // Training state teardown (train.hip), called by nml_model_destroy.
 void train_release(nml_model* m);
-// Parameters change, or a caller gets a pointer to them: a backward of the last loss forms its
-// logits from the parameters that it finds.
+// Parameters change, or a caller first gets a pointer to them: a backward of the last loss
+// forms its logits from the parameters that it finds.
 void train_params_open(nml_model* m);
 // After a parameter upload: an fp16 model's AdamW master copy of that parameter (when the
 // optimizer state exists) is taken again from the uploaded values.

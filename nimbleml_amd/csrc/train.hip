@@ -39,6 +39,8 @@ struct TrainState {
   int B = 0, S = 0;
   bool saved = false;
   bool logits_kept = false;  // `logits` holds them and no backward has used them up
+  bool emb_summed = false;   // emb_sum holds the checksum of the head that formed them
+  uint64_t emb_sum = 0;
   int what = 0;        // the saved forward: kSavedLoss, kSavedBlocks or kSavedMha
   int final_norm = 0;  // kSavedBlocks: the final RMSNorm ran after the blocks
   int full = 0;        // module forwards: non-causal attention
@@ -129,6 +131,48 @@ int ensure_train(nml_model* m) {
 
 // Logits of a training forward kept for its backward: up to 4 GiB of the card's 288.
 constexpr size_t kKeptLogits = (size_t)4 << 30;
+
+// Checksum of n 16-byte pieces: the sum over 64-bit words of a mix of the word and its place
+// (splitmix64's finaliser), the same in any order.
+__device__ __forceinline__ uint64_t mix64(uint64_t x) {
+  x = (x ^ (x >> 30)) * 0xbf58476d1ce4e5b9ull;
+  x = (x ^ (x >> 27)) * 0x94d049bb133111ebull;
+  return x ^ (x >> 31);
+}
+
+__global__ __launch_bounds__(256) void checksum_kernel(const ulonglong2* __restrict__ p, size_t n,
+                                                       unsigned long long* __restrict__ out) {
+  constexpr int U = 4;  // loads in flight
+  const size_t step = static_cast<size_t>(gridDim.x) * 256;
+  uint64_t s = 0;
+  for (size_t i = blockIdx.x * 256ull + threadIdx.x; i < n; i += U * step) {
+    ulonglong2 v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = p[i + u * step < n ? i + u * step : i];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (i + u * step < n) {
+        const uint64_t at = 2 * (i + u * step) + 1;
+        s += mix64(v[u].x + at * 0x9e3779b97f4a7c15ull) + mix64(v[u].y + (at + 1) * 0x9e3779b97f4a7c15ull);
+      }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(static_cast<unsigned long long>(s), o, 64);
+  __shared__ uint64_t part[4];
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) atomicAdd(out, static_cast<unsigned long long>(part[0] + part[1] + part[2] + part[3]));
+}
+
+// The checksum of the token embedding (rows of whole 16-byte pieces, as the products need) added
+// to *out, in stream order.
+int embedding_checksum(const nml_model* m, unsigned long long* out, hipStream_t st) {
+  const size_t n = (size_t)m->V * m->d * m->es / 16, blocks = (n + 1023) / 1024;
+  checksum_kernel<<<static_cast<unsigned>(blocks < 512 ? blocks : 512), 256, 0, st>>>(
+      static_cast<const ulonglong2*>(m->emb), n, out);
+  NML_LAUNCHED();
+  return 0;
+}
 
 // Rows per logits chunk: at most 512 MiB of logits at once.
 size_t logits_chunk(const nml_model* m, size_t R) {
@@ -455,12 +499,12 @@ int nml_model_loss_train(nml_model* m, const int64_t* ids, const int64_t* labels
   int64_t* dids = reinterpret_cast<int64_t*>(io);
   int64_t* dlab = reinterpret_cast<int64_t*>(io + ib);
   int* err = reinterpret_cast<int*>(io + 2 * ib);
-  double* acc = reinterpret_cast<double*>(io + 2 * ib + 256);
+  double* acc = reinterpret_cast<double*>(io + 2 * ib + 256);  // Σ loss, rows, mean; two checksums
   float* row_loss = reinterpret_cast<float*>(io + 2 * ib + 512);
   int* row_valid = reinterpret_cast<int*>(io + 2 * ib + 512 + rb);
   NML_HIP(hipMemcpyAsync(dids, ids, (size_t)R * 8, hipMemcpyDeviceToDevice, st));
   NML_HIP(hipMemcpyAsync(dlab, labels, (size_t)R * 8, hipMemcpyDeviceToDevice, st));
-  NML_HIP(hipMemsetAsync(err, 0, sizeof(int), st));
+  NML_HIP(hipMemsetAsync(err, 0, 512, st));
 
   NML_TRY(launch_embed(dt, dids, m->emb, posw(m), nullptr, sv.x, B, S, d, m->V, m->P, err, st));
   NML_TRY(blocks_forward_saving(m, sv, B, S, MaskMode{}, st));
@@ -484,11 +528,18 @@ int nml_model_loss_train(nml_model* m, const int64_t* ids, const int64_t* labels
     NML_TRY(launch_ce_reduce(row_loss, row_valid, n, acc, r0 > 0, st));
   }
   NML_TRY(launch_ce_finalize(acc, acc + 2, st));
-  double host[3];
-  int herr = 0;
-  NML_HIP(hipMemcpyAsync(host, acc, sizeof(host), hipMemcpyDeviceToHost, st));
-  NML_HIP(hipMemcpyAsync(&herr, err, sizeof(int), hipMemcpyDeviceToHost, st));
+  // A caller with a pointer into the parameters may write the head before the backward, which
+  // then has to form the logits again; the checksum tells (a changed head passes for the same
+  // one in 2^64). Both checksums, the copy and the wait cost a d 1024, V 32000 step 56 µs (float32
+  // 130) of the 277 and 1573 above, and the d 256, V 4096 step 43.
+  const bool summed = keep && m->params_out;
+  if (summed) NML_TRY(embedding_checksum(m, reinterpret_cast<unsigned long long*>(acc + 3), st));
+  double words[36], *host = words + 32;  // the error word, 256 bytes later the accumulators
+  NML_HIP(hipMemcpyAsync(words, err, sizeof(words), hipMemcpyDeviceToHost, st));
   NML_HIP(hipStreamSynchronize(st));
+  int herr = 0;
+  std::memcpy(&herr, words, sizeof(herr));
+  std::memcpy(&t->emb_sum, host + 3, sizeof(t->emb_sum));
   NML_REQUIRE((herr & 1) == 0, "Token ID out of range [0, %d)", m->V);
   NML_REQUIRE((herr & 2) == 0, "label out of range [0, %d)", m->V);
   *loss = host[2];
@@ -499,6 +550,7 @@ int nml_model_loss_train(nml_model* m, const int64_t* ids, const int64_t* labels
   t->n_valid = host[1];
   t->what = kSavedLoss;
   t->logits_kept = keep;
+  t->emb_summed = summed;
   t->saved = true;
   t->generation += 1;
   return 0;
@@ -530,8 +582,17 @@ int nml_model_backward(nml_model* m, double grad_scale) {
   // tied head + cross-entropy, chunk by chunk; dH lands in DX
   const float scale = static_cast<float>(grad_scale / t->n_valid);
   const size_t chunk = logits_chunk(m, R);
-  const bool kept = t->logits_kept;  // (a second backward of this loss forms them again)
+  bool kept = t->logits_kept;  // (a second backward of this loss forms them again)
   t->logits_kept = false;
+  if (kept && t->emb_summed) {
+    // (the second slot, cleared by the loss; the logits are kept for one backward only)
+    unsigned long long* sum = reinterpret_cast<unsigned long long*>(static_cast<char*>(t->io.p) + 2 * ib + 256) + 4;
+    uint64_t now = 0;
+    NML_TRY(embedding_checksum(m, sum, st));
+    NML_HIP(hipMemcpyAsync(&now, sum, sizeof(now), hipMemcpyDeviceToHost, st));
+    NML_HIP(hipStreamSynchronize(st));
+    kept = now == t->emb_sum;
+  }
   if (!kept) NML_TRY(m->logits_ws.ensure(align256(chunk * V * es)));
   for (size_t r0 = 0; r0 < (size_t)R; r0 += chunk) {
     const int n = (int)(((size_t)R - r0 < chunk) ? (size_t)R - r0 : chunk);

@@ -72,3 +72,47 @@ def test_second_backward_of_a_loss_equals_the_first(dtype):
     set_head(2)
     for x, y in zip(backward(), changed):
         assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
+@pytest.mark.parametrize("vocab,d", [(512, 64), (20000, 128)])
+def test_head_written_through_an_earlier_pointer(vocab, d, dtype):
+    """Between a loss and its backward the head changes in one element, through a pointer taken
+    before the loss: the gradients are those of a backward that forms the logits itself."""
+    import nimbleml_amd as nm
+    from oracle.weights import GPTConfig, make_weights, random_ids
+
+    cfg = GPTConfig(vocab, d, 4, 1, 16)
+    w = make_weights(cfg, seed=3, dtype=dtype, rich=True)
+    m = nm.GPT.from_arrays(w, cfg.vocab_size, cfg.d_model, cfg.num_heads, cfg.num_layers,
+                           cfg.max_seq_len, dtype=dtype)
+    ids, lab = random_ids((2, 9), vocab, seed=5), random_ids((2, 9), vocab, seed=6)
+    h, loss, ptr = m._device_model(), C.c_double(), C.c_void_p()
+    dids, dlab = N.DeviceArray.from_host(ids), N.DeviceArray.from_host(lab)
+    head = np.ascontiguousarray(w["token_emb.weights"])
+    other = head.copy()
+    other[-1, -1] += np.asarray(4, dtype)
+
+    def backward():
+        N.check(N.lib.nml_model_zero_grad(h))
+        N.check(N.lib.nml_model_backward(h, 1.0))
+        return [m._grad_array(k, 0, m._device_shape(k)) for k in (N.P_TOKEN_EMB, N.P_LN_F, N.P_W1)]
+
+    def loss_train():
+        N.check(N.lib.nml_model_loss_train(h, dids.ptr, dlab.ptr, 2, 9, 0, 0, C.byref(loss)))
+
+    loss_train()
+    plain = backward()
+    N.check(N.lib.nml_model_set_param(h, N.P_TOKEN_EMB, 0, other.ctypes.data, other.nbytes))
+    want = backward()  # of the first loss, with the other head
+    assert not np.array_equal(want[0], plain[0])
+    N.check(N.lib.nml_model_set_param(h, N.P_TOKEN_EMB, 0, head.ctypes.data, head.nbytes))
+    N.check(N.lib.nml_model_param_ptr(h, N.P_TOKEN_EMB, 0, C.byref(ptr)))
+    loss_train()
+    N.check(N.lib.nml_memcpy_h2d(ptr, other.ctypes.data, other.nbytes))
+    for x, y in zip(backward(), want):
+        assert np.array_equal(x, y)
+    N.check(N.lib.nml_memcpy_h2d(ptr, head.ctypes.data, head.nbytes))
+    loss_train()
+    for x, y in zip(backward(), plain):
+        assert np.array_equal(x, y)
