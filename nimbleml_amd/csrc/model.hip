@@ -110,7 +110,7 @@ int acts_in(nml_model* m, Buf& buf, int R, int Bdec, Acts* a) {
   const size_t rf = align256((size_t)R * m->F * m->es);
   const size_t part = Bdec ? align256(attention_decode_workspace(Bdec, m->H, m->dk, m->P)) : 0;
   const size_t ssq = Bdec ? align256((size_t)Bdec * (m->d / 16 + 1) * sizeof(float)) : 0;
-  NML_TRY(buf.ensure(4 * rd + rf + part + ssq));
+  NML_TRY(ensure(m, buf, 4 * rd + rf + part + ssq));
   char* b = static_cast<char*>(buf.p);
   a->x = b;
   a->xn = b + rd;
@@ -135,7 +135,7 @@ struct Small {
 
 int small_for(nml_model* m, int B, Small* s) {
   const size_t need = 256 + 256 + 3 * align256((size_t)B * 4 + 4);
-  NML_TRY(m->small.ensure(need < 4096 ? 4096 : need));
+  NML_TRY(ensure(m, m->small, need < 4096 ? 4096 : need));
   char* b = static_cast<char*>(m->small.p);
   s->err = reinterpret_cast<int*>(b);
   s->acc = reinterpret_cast<double*>(b + 256);
@@ -484,7 +484,7 @@ int persist_prepare(nml_model* m, const int64_t* ids, int64_t* tok, int* err, Pe
   pa->b2 = l0.b2;
   pa->layer_bytes = stride;
   const size_t sb = align256(persist_slot_count(m->d, m->H) * 8);
-  NML_TRY(m->persist.ensure(sb + 256));
+  NML_TRY(ensure(m, m->persist, sb + 256));
   char* base = static_cast<char*>(m->persist.p);
   uint32_t* epoch = reinterpret_cast<uint32_t*>(base + sb);
   persist_begin_kernel<<<clear_grid(sb / 4), 256, 0, st>>>(reinterpret_cast<uint32_t*>(base), sb / 4, epoch, ids, tok,
@@ -620,7 +620,7 @@ int prefill_rows(nml_model* m, nml_cache* c, const int64_t* prompts, size_t prom
     std::vector<int32_t> starts(B);
     for (int b = 0, r = 0; b < B; r += plen[b], ++b) starts[b] = r;
     tab.insert(tab.end(), starts.begin(), starts.end());
-    NML_TRY(m->ragged.ensure(tab.size() * 4));
+    NML_TRY(ensure(m, m->ragged, tab.size() * 4));
     const int32_t* dtab = static_cast<const int32_t*>(m->ragged.p);
     NML_HIP(hipMemcpyAsync(m->ragged.p, tab.data(), tab.size() * 4, hipMemcpyHostToDevice, st));
     const Ragged rg{dtab, dtab + R, dtab + R + B, R};
@@ -794,7 +794,7 @@ int nml_model_forward(nml_model* m, const int64_t* ids, size_t batch, size_t seq
   Acts a;
   NML_TRY(acts_for(m, B * S, 0, &a));
   const size_t kvb = align256((size_t)B * S * m->d * m->es);
-  NML_TRY(m->kvs.ensure(2 * kvb));
+  NML_TRY(ensure(m, m->kvs, 2 * kvb));
   void* kbuf = m->kvs.p;
   void* vbuf = static_cast<char*>(m->kvs.p) + kvb;
   NML_TRY(launch_embed(m->dt, ids, m->emb, posw(m), nullptr, a.x, B, S, m->d, m->V, m->P, nullptr,
@@ -817,7 +817,7 @@ int nml_model_blocks_forward(nml_model* m, const void* x, void* out, size_t batc
   NML_TRY(acts_for(m, B * S, 0, &a));
   const size_t bytes = (size_t)B * S * m->d * m->es;
   const size_t kvb = align256(bytes);
-  NML_TRY(m->kvs.ensure(2 * kvb));
+  NML_TRY(ensure(m, m->kvs, 2 * kvb));
   void* kbuf = m->kvs.p;
   void* vbuf = static_cast<char*>(m->kvs.p) + kvb;
   NML_HIP(hipMemcpyAsync(a.x, x, bytes, hipMemcpyDeviceToDevice, st));
@@ -844,7 +844,7 @@ int nml_model_mha_forward(nml_model* m, int layer, const void* x, void* out, siz
   Acts a;
   NML_TRY(acts_for(m, B * S, 0, &a));
   const size_t kvb = align256((size_t)B * S * m->d * m->es);
-  NML_TRY(m->kvs.ensure(2 * kvb));
+  NML_TRY(ensure(m, m->kvs, 2 * kvb));
   AttnMode am;
   am.full = causal ? 0 : 1;
   am.mask = mask;
@@ -883,7 +883,7 @@ int nml_model_loss(nml_model* m, const int64_t* ids, const int64_t* labels, size
   Acts a;
   NML_TRY(acts_for(m, R, 0, &a));
   const size_t kvb = align256((size_t)R * m->d * m->es);
-  NML_TRY(m->kvs.ensure(2 * kvb));
+  NML_TRY(ensure(m, m->kvs, 2 * kvb));
   void* kbuf = m->kvs.p;
   void* vbuf = static_cast<char*>(m->kvs.p) + kvb;
   Small sm;
@@ -899,7 +899,7 @@ int nml_model_loss(nml_model* m, const int64_t* ids, const int64_t* labels, size
     const int tn = (m->V + kLinearCETile - 1) / kLinearCETile;
     const size_t pb = align256((size_t)R * tn * sizeof(float2));
     const size_t rb = align256((size_t)R * 4);
-    NML_TRY(m->logits_ws.ensure(pb + 3 * rb));
+    NML_TRY(ensure(m, m->logits_ws, pb + 3 * rb));
     char* w = static_cast<char*>(m->logits_ws.p);
     float2* part = reinterpret_cast<float2*>(w);
     float* label_logit = reinterpret_cast<float*>(w + pb);
@@ -925,7 +925,7 @@ int nml_model_loss(nml_model* m, const int64_t* ids, const int64_t* labels, size
   while (chunk > 1 && chunk * m->V * m->es > ((size_t)512 << 20)) chunk = (chunk + 1) / 2;
   const size_t lb = align256(chunk * m->V * m->es);
   const size_t rb = align256((size_t)R * 4);
-  NML_TRY(m->logits_ws.ensure(lb + 2 * rb));
+  NML_TRY(ensure(m, m->logits_ws, lb + 2 * rb));
   void* lg = m->logits_ws.p;
   float* row_loss = reinterpret_cast<float*>(static_cast<char*>(m->logits_ws.p) + lb);
   int* row_valid = reinterpret_cast<int*>(static_cast<char*>(m->logits_ws.p) + lb + rb);
@@ -956,9 +956,13 @@ int nml_cache_create(nml_model* m, size_t batch, nml_cache** out) {
   c->m = m;
   c->B = (int)batch;
   const size_t bytes = (size_t)m->L * batch * m->H * m->P * m->dk * m->es;
-  hipError_t e1 = hipMalloc(&c->k, bytes);
-  hipError_t e2 = e1 == hipSuccess ? hipMalloc(&c->v, bytes) : e1;
-  hipError_t e3 = e2 == hipSuccess ? hipMalloc(&c->len_dev, align256(batch * 4)) : e2;
+  auto room = [m](auto** p, size_t n) {
+    const hipError_t e = hipMalloc(p, n);
+    return e != hipSuccess && train_drop_logits(m) ? hipMalloc(p, n) : e;
+  };
+  hipError_t e1 = room(&c->k, bytes);
+  hipError_t e2 = e1 == hipSuccess ? room(&c->v, bytes) : e1;
+  hipError_t e3 = e2 == hipSuccess ? room(&c->len_dev, align256(batch * 4)) : e2;
   if (e3 != hipSuccess) {
     set_error("cache: allocation of 2 × %zu bytes failed: %s", bytes, hipGetErrorString(e3));
     if (c->k) (void)hipFree(c->k);
@@ -1116,7 +1120,7 @@ int nml_model_generate(nml_model* m, const int64_t* prompts, size_t prompt_strid
 
   // Logits for the batch (B, V).
   const size_t lb = align256((size_t)B * m->V * m->es);
-  NML_TRY(m->logits_ws.ensure(lb));
+  NML_TRY(ensure(m, m->logits_ws, lb));
   void* logits = m->logits_ws.p;
 
   NML_TRY(prefill_rows(m, c, prompts, prompt_stride, plen, sm, logits, st));

@@ -84,6 +84,16 @@ inline const void* posw(const nml_model* m) { return rope_on(m) ? nullptr : m->p
 
 int check_ready(nml_model* m);
 
+// Gives back the logits that a training loss keeps (none are needed: a backward without them
+// forms them again). True: there were some.
+bool train_drop_logits(nml_model* m);
+// Room in one of the model's buffers; where the device has none left, the kept logits make it.
+inline int ensure(nml_model* m, Buf& b, size_t want) {
+  if (b.ensure(want) == 0) return 0;
+  if (!train_drop_logits(m)) return -1;
+  return b.ensure(want);
+}
+
 // Training state teardown (train.hip), called by nml_model_destroy.
 void train_release(nml_model* m);
 // Parameters change, or a caller first gets a pointer to them: a backward of the last loss

@@ -123,14 +123,24 @@ int ensure_train(nml_model* m) {
   if (!m->train) m->train = new TrainState();
   TrainState* t = m->train;
   if (!t->grads.p) {
-    NML_TRY(t->grads.ensure(f32_bytes(m)));
+    NML_TRY(ensure(m, t->grads, f32_bytes(m)));
     NML_HIP(hipMemsetAsync(t->grads.p, 0, f32_bytes(m), nml::stream()));
   }
   return 0;
 }
 
-// Logits of a training forward kept for its backward: up to 4 GiB of the card's 288.
+// Logits of a training forward are kept for its backward up to 4 GiB, and where that leaves at
+// least 7/8 of the memory that is free: the backward's own scratch comes after them.
 constexpr size_t kKeptLogits = (size_t)4 << 30;
+
+bool keep_logits(TrainState* t, size_t bytes) {
+  if (bytes <= t->logits.bytes) return true;
+  size_t free = 0, total = 0;
+  if (bytes > kKeptLogits || hipMemGetInfo(&free, &total) != hipSuccess || bytes > free / 8) return false;
+  if (t->logits.ensure(bytes) == 0) return true;
+  (void)hipGetLastError();  // no room is no error
+  return false;
+}
 
 // Checksum of n 16-byte pieces: the sum over 64-bit words of a mix of the word and its place
 // (splitmix64's finaliser), the same in any order.
@@ -235,11 +245,11 @@ int ensure_adam(nml_model* m) {
   hipStream_t st = nml::stream();
   const size_t fb = f32_bytes(m);
   if (!t->moments.p) {
-    NML_TRY(t->moments.ensure(2 * fb));
+    NML_TRY(ensure(m, t->moments, 2 * fb));
     NML_HIP(hipMemsetAsync(t->moments.p, 0, 2 * fb, st));
   }
   if (m->dt == F16 && !t->masters.p) {
-    NML_TRY(t->masters.ensure(fb));
+    NML_TRY(ensure(m, t->masters, fb));
     NML_TRY(launch_convert(F16, m->arena, F32, t->masters.p, m->arena_bytes / m->es, st));
   }
   return 0;
@@ -335,7 +345,7 @@ int bwd_scratch(nml_model* m, int B, int S, BwdScratch* w) {
   const size_t pn = (size_t)(rmsnorm_bwd_parts(R) > colsum_parts(R) ? rmsnorm_bwd_parts(R)
                                                                      : colsum_parts(R)) *
                     widest;
-  NML_TRY(m->train->scratch.ensure(2 * rd + r3 + rf + rv + align256(pn * 4)));
+  NML_TRY(ensure(m, m->train->scratch, 2 * rd + r3 + rf + rv + align256(pn * 4)));
   char* sp = static_cast<char*>(m->train->scratch.p);
   w->G = sp;
   w->DX = sp + rd;
@@ -421,7 +431,7 @@ int module_mask(nml_model* m, int S, int causal, const void* mask, hipStream_t s
   t->masked = mask != nullptr;
   if (mask && S > 0) {
     const size_t bytes = (size_t)S * S * m->es;
-    NML_TRY(t->mask.ensure(bytes));
+    NML_TRY(ensure(m, t->mask, bytes));
     NML_HIP(hipMemcpyAsync(t->mask.p, mask, bytes, hipMemcpyDeviceToDevice, st));
     mm->mask = t->mask.p;
   }
@@ -439,6 +449,15 @@ MaskMode saved_mask(const TrainState* t) {
 
 void train_params_open(nml_model* m) {
   if (m->train) m->train->logits_kept = false;
+}
+
+bool train_drop_logits(nml_model* m) {
+  if (!m->train || !m->train->logits.p) return false;
+  (void)hipGetLastError();  // the allocation that failed
+  (void)hipStreamSynchronize(nml::stream());
+  m->train->logits.release();
+  m->train->logits_kept = false;
+  return true;
 }
 
 int train_param_uploaded(nml_model* m, const void* param, size_t elems) {
@@ -490,11 +509,11 @@ int nml_model_loss_train(nml_model* m, const int64_t* ids, const int64_t* labels
   }
   hipStream_t st = nml::stream();
   Saved sv;
-  NML_TRY(t->acts.ensure(saved_bytes(m, B, S, nullptr, nullptr)));
+  NML_TRY(ensure(m, t->acts, saved_bytes(m, B, S, nullptr, nullptr)));
   saved_bytes(m, B, S, &sv, static_cast<char*>(t->acts.p));
   // io: ids, labels, then err / loss accumulators, per-row loss and validity
   const size_t ib = align256((size_t)R * 8), rb = align256((size_t)R * 4);
-  NML_TRY(t->io.ensure(2 * ib + 512 + 2 * rb));
+  NML_TRY(ensure(m, t->io, 2 * ib + 512 + 2 * rb));
   char* io = static_cast<char*>(t->io.p);
   int64_t* dids = reinterpret_cast<int64_t*>(io);
   int64_t* dlab = reinterpret_cast<int64_t*>(io + ib);
@@ -510,14 +529,13 @@ int nml_model_loss_train(nml_model* m, const int64_t* ids, const int64_t* labels
   NML_TRY(blocks_forward_saving(m, sv, B, S, MaskMode{}, st));
   NML_TRY(launch_rmsnorm(dt, sv.xl, m->lnf, sv.hf, nullptr, nullptr, R, d, kEps, st));
 
-  // The logits stay for the backward, which forms their gradient in place, where they are at
-  // most kKeptLogits bytes and there is room for them; else they are formed chunk by chunk,
+  // The logits stay for the backward, which forms their gradient in place, where there is ample
+  // room for them (keep_logits); else they are formed chunk by chunk,
   // here and in the backward. (Forming them again cost a d 1024, V 32000, 4 × 1024 step 277 µs
   // in fp16 and 1573 in float32.)
   const size_t chunk = logits_chunk(m, R), all = (size_t)R * m->V * es;
-  const bool keep = all <= kKeptLogits && t->logits.ensure(align256(all)) == 0;
-  if (!keep) (void)hipGetLastError();  // no room is no error
-  if (!keep) NML_TRY(m->logits_ws.ensure(align256(chunk * m->V * es)));
+  const bool keep = keep_logits(t, align256(all));
+  if (!keep) NML_TRY(ensure(m, m->logits_ws, align256(chunk * m->V * es)));
   for (size_t r0 = 0; r0 < (size_t)R; r0 += chunk) {
     const int n = (int)(((size_t)R - r0 < chunk) ? (size_t)R - r0 : chunk);
     void* lg = keep ? static_cast<char*>(t->logits.p) + r0 * m->V * es : m->logits_ws.p;
@@ -593,7 +611,7 @@ int nml_model_backward(nml_model* m, double grad_scale) {
     NML_HIP(hipStreamSynchronize(st));
     kept = now == t->emb_sum;
   }
-  if (!kept) NML_TRY(m->logits_ws.ensure(align256(chunk * V * es)));
+  if (!kept) NML_TRY(ensure(m, m->logits_ws, align256(chunk * V * es)));
   for (size_t r0 = 0; r0 < (size_t)R; r0 += chunk) {
     const int n = (int)(((size_t)R - r0 < chunk) ? (size_t)R - r0 : chunk);
     const char* h = sv.hf + r0 * d * es;
@@ -626,10 +644,10 @@ int nml_model_logits_backward(nml_model* m, const int64_t* ids, size_t batch, si
   if (R == 0) return 0;
   hipStream_t st = nml::stream();
   Saved sv;
-  NML_TRY(t->acts.ensure(saved_bytes(m, B, S, nullptr, nullptr)));
+  NML_TRY(ensure(m, t->acts, saved_bytes(m, B, S, nullptr, nullptr)));
   saved_bytes(m, B, S, &sv, static_cast<char*>(t->acts.p));
   const size_t ib = align256((size_t)R * 8);
-  NML_TRY(t->io.ensure(ib + 256));
+  NML_TRY(ensure(m, t->io, ib + 256));
   int64_t* dids = reinterpret_cast<int64_t*>(t->io.p);
   int* err = reinterpret_cast<int*>(static_cast<char*>(t->io.p) + ib);
   NML_HIP(hipMemcpyAsync(dids, ids, (size_t)R * 8, hipMemcpyDeviceToDevice, st));
@@ -668,7 +686,7 @@ static int module_forward_begin(nml_model* m, size_t batch, size_t seq, int caus
   TrainState* t = m->train;
   t->saved = false;
   const int B = (int)batch, S = (int)seq;
-  NML_TRY(t->acts.ensure(saved_bytes(m, B, S, nullptr, nullptr)));
+  NML_TRY(ensure(m, t->acts, saved_bytes(m, B, S, nullptr, nullptr)));
   saved_bytes(m, B, S, sv, static_cast<char*>(t->acts.p));
   NML_TRY(module_mask(m, S, causal, mask, nml::stream(), mm));
   t->B = B;

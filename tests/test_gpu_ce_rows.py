@@ -116,3 +116,66 @@ def test_head_written_through_an_earlier_pointer(vocab, d, dtype):
     loss_train()
     for x, y in zip(backward(), plain):
         assert np.array_equal(x, y)
+
+
+def allocate(size):
+    """A device block of that many bytes, or None."""
+    p = C.c_void_p()
+    return p.value if N.lib.nml_malloc(size, C.byref(p)) == 0 else None
+
+
+def fill_memory(left):
+    """Blocks that take the device's memory but for `left` bytes."""
+    spare, blocks, size = allocate(left), [], 1 << 36
+    while size >= 1 << 24:
+        block = allocate(size)
+        if block is None:
+            size //= 2
+        else:
+            blocks.append(block)
+    N.check(N.lib.nml_free(spare))
+    x = N.DeviceArray.from_host(np.zeros(8, np.float32))
+    N.lib.nml_gelu_forward_device(x.ptr, x.ptr, None, 8, N.F32)  # takes the last allocation's error
+    return blocks
+
+
+def release(blocks):
+    for p in blocks:
+        N.check(N.lib.nml_free(p))
+
+
+@pytest.mark.parametrize("left", [48 << 20, 4 << 30])
+def test_kept_logits_give_way(left):
+    """With less memory left after the loss than the backward's scratch, the logits kept for it
+    make the room; with little left before the loss, none are kept."""
+    import nimbleml_amd as nm
+    from oracle.weights import GPTConfig, make_weights, random_ids
+
+    cfg, rows, seq = GPTConfig(50000, 512, 4, 1, 512), 8, 512
+    w = make_weights(cfg, seed=3, dtype=np.float32)
+    ids, lab = (random_ids((rows, seq), cfg.vocab_size, seed=s) for s in (5, 6))
+    logits = rows * seq * cfg.vocab_size * 4  # 819 MB; half of it at a time without keeping them
+    early = left > logits
+    got = []
+    for tight in (False, True):
+        m = nm.GPT.from_arrays(w, cfg.vocab_size, cfg.d_model, cfg.num_heads, cfg.num_layers, cfg.max_seq_len,
+                               dtype=np.float32)
+        h, loss = m._device_model(), C.c_double()
+        dids, dlab = N.DeviceArray.from_host(ids), N.DeviceArray.from_host(lab)
+        N.check(N.lib.nml_model_zero_grad(h))
+        blocks = fill_memory(left) if tight and early else []
+        N.check(N.lib.nml_model_loss_train(h, dids.ptr, dlab.ptr, rows, seq, 0, 0, C.byref(loss)))
+        if tight and early:  # the activations are 140 MB
+            probe = allocate(left - 140 * 2**20 - logits * 3 // 4)
+            assert probe is not None
+            release([probe])
+        elif tight:
+            blocks = fill_memory(left)
+        try:
+            N.check(N.lib.nml_model_backward(h, 1.0))
+        finally:
+            release(blocks)
+        got.append([m._grad_array(k, 0, m._device_shape(k)) for k in (N.P_TOKEN_EMB, N.P_LN_F, N.P_WQKV, N.P_B2)])
+        del m
+    for x, y in zip(*got):  # (a weight gradient over two chunks sums in another order)
+        assert np.abs(x - y).max() <= 1e-5 * np.abs(x).max()
