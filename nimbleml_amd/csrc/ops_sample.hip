@@ -590,7 +590,7 @@ __device__ int find_nth(int V, int j, FP pred, Shared& sh) {
 // spread over hundreds of them, so the LDS atomics seldom meet), a scan of the bins, and the
 // walk order inside the bin that the target falls into. Sums over the row are taken as the
 // general path takes them. Declines (the general path then runs) when that bin holds more
-// than kBinCand elements, as a row of equal or of no logits does.
+// than kBinCand elements, as a row of equal logits does, and when the probabilities are NaN.
 // 32 rows of 32000 fp16 logits, top-p 0.9: 377 µs on the general path (about 20 passes of
 // exponentials and divisions, and LDS atomics on the few bins that the leading byte of a
 // probability can fall into), 94 here.
@@ -724,6 +724,7 @@ __device__ int sample_topp_regs(const Row<T>& row, int k, double top_p, double u
       se += x[j];
     }
   se = block_sum_f(se, sh);
+  if (!__builtin_isfinite(se)) return -1;  // an infinite or NaN logit, or no finite one: no order to walk
 #pragma unroll
   for (int j = 0; j < E; ++j) x[j] = held(j) ? x[j] / se : 0.f;  // x now holds the probabilities
   auto keyp = [&](int j) { return fkey(x[j]); };

@@ -56,3 +56,19 @@ def test_masked_tokens():
     lg[:, 7:2990] = -np.inf
     check(lg, 0, 0.9, np.array([0.03, 0.31, 0.62, 0.97]))
     check(lg, 5, 0.9, np.array([0.03, 0.31, 0.62, 0.97]))
+
+
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
+@pytest.mark.parametrize("vocab", [40, 1000, 1024, 3000])
+@pytest.mark.parametrize("top_k", [0, 7])
+def test_rows_without_probabilities(vocab, top_k, dtype):
+    """Rows whose probabilities are NaN (a NaN or infinite logit, no finite logit) give the last
+    token whatever the vocabulary, as a walk over one tied key does; a row beside them is its own."""
+    r = np.random.RandomState(vocab)
+    lg = r.randn(4, vocab).astype(dtype)
+    lg[0, 5], lg[1, 6] = np.nan, np.inf
+    lg[2] = -np.inf
+    got = K.sample_tokens(lg, temperature=0.8, top_k=top_k, top_p=0.9, uniforms=np.full(4, 0.5))
+    alone = K.sample_tokens(lg[3:], temperature=0.8, top_k=top_k, top_p=0.9, uniforms=np.full(1, 0.5))
+    assert (got[:3] == vocab - 1).all(), got
+    assert got[3] == alone[0]
