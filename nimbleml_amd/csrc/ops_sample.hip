@@ -593,7 +593,7 @@ __device__ int find_nth(int V, int j, FP pred, Shared& sh) {
 // than kBinCand elements, as a row of equal logits does, and when the probabilities are NaN.
 // 32 rows of 32000 fp16 logits, top-p 0.9: 377 µs on the general path (about 20 passes of
 // exponentials and divisions, and LDS atomics on the few bins that the leading byte of a
-// probability can fall into), 94 here.
+// probability can fall into), 82 here (24 of the 128 registers spilled).
 constexpr int kBinBits = 12, kBins = 1 << kBinBits, kBinShift = 16, kBinCand = 1024;
 
 struct BinCand {
@@ -618,7 +618,7 @@ __device__ __forceinline__ float key_value(uint32_t k) {
 // in(j) whose inclusive running weight exceeds target; the walk's last if none does. top: a
 // key no element exceeds. False: declined.
 template <int E, typename FK, typename FW, typename FI>
-__device__ bool walk_to(uint32_t top, double target, FK key_of, FW weight, FI in, Shared& sh, BinWork& bw,
+__device__ __forceinline__ bool walk_to(uint32_t top, double target, FK key_of, FW weight, FI in, Shared& sh, BinWork& bw,
                         uint32_t* key, int* index) {
   const int tid = threadIdx.x;
   __syncthreads();  // the previous walk's readers are done
@@ -694,7 +694,7 @@ __device__ bool walk_to(uint32_t top, double target, FK key_of, FW weight, FI in
 }
 
 template <typename T, int E>
-__device__ int sample_topp_regs(const Row<T>& row, int k, double top_p, double u, Shared& sh, BinWork& bw) {
+__device__ __forceinline__ int sample_topp_regs(const Row<T>& row, int k, double top_p, double u, Shared& sh, BinWork& bw) {
   const int tid = threadIdx.x, V = row.V;
   float x[E];
   float mx = -INFINITY;
@@ -765,7 +765,13 @@ __device__ int sample_topp_regs(const Row<T>& row, int k, double top_p, double u
 constexpr int kRowCacheBytes = 100 * 1024 + 512;
 static_assert(sizeof(BinWork) <= kRowCacheBytes, "the top-p walk works in the row cache");
 
-template <typename T>
+__host__ __device__ inline bool topp_of(const SampleArgs& a) { return a.top_p > 0.f && a.top_p < 1.f; }
+
+// REGS > 0: top-p, with or without top-k, from registers, REGS elements a thread; 0: every other
+// call. Kernels of their own: the register form's frame (128 registers, the most that 1024 threads
+// leave each, and scratch for the general path that it falls back on) cost greedy, top-k and plain
+// rows 0.8 µs a call.
+template <typename T, int REGS>
 __global__ __launch_bounds__(kThreads) void sample_kernel(SampleArgs a) {
   __shared__ Shared sh;
   __shared__ __attribute__((aligned(16))) char s_row[kRowCacheBytes];
@@ -795,8 +801,8 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(SampleArgs a) {
     __syncthreads();
   }
 
-  const bool sampled = a.temperature > 0.f;
-  const bool use_p = a.top_p > 0.f && a.top_p < 1.f;
+  const bool sampled = REGS > 0 || a.temperature > 0.f;
+  const bool use_p = REGS > 0 || topp_of(a);
   const bool use_k = a.top_k > 0;
   const int k_eff = a.top_k < V ? a.top_k : V;
   double u = 0.0;
@@ -809,11 +815,9 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(SampleArgs a) {
     if (sampled && use_k && !use_p && sample_regs_applies(row, k_eff))
       chosen = sample_topk_regs(row, k_eff, u, sh, s_cand, s_candx);
   }
-  if (sampled && use_p && V <= 50 * kThreads) {
+  if constexpr (REGS > 0) {
     BinWork& bw = *reinterpret_cast<BinWork*>(s_row);
-    const int k = use_k ? k_eff : 0;
-    chosen = V <= 32 * kThreads ? sample_topp_regs<T, 32>(row, k, static_cast<double>(a.top_p), u, sh, bw)
-                                : sample_topp_regs<T, 50>(row, k, static_cast<double>(a.top_p), u, sh, bw);
+    chosen = sample_topp_regs<T, REGS>(row, use_k ? k_eff : 0, static_cast<double>(a.top_p), u, sh, bw);
     __syncthreads();
   }
   if (chosen < 0) {
@@ -993,6 +997,26 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(SampleArgs a) {
   }
 }
 
+template <typename T>
+int sample_launch(const SampleArgs& a, hipStream_t st) {
+  // As many elements a thread as the vocabulary needs (32 rows of 1000 logits: 22.6 µs with 4, 37.2
+  // with 32), up to 50: a thread then spills 175 registers (32 rows of 50304 logits: 158 µs, the
+  // general path 538), and longer rows take the general path.
+  const int per = (a.V + kThreads - 1) / kThreads;
+  if (a.temperature <= 0.f || !topp_of(a) || per > 50)
+    sample_kernel<T, 0><<<a.B, kThreads, 0, st>>>(a);
+  else if (per <= 4)
+    sample_kernel<T, 4><<<a.B, kThreads, 0, st>>>(a);
+  else if (per <= 16)
+    sample_kernel<T, 16><<<a.B, kThreads, 0, st>>>(a);
+  else if (per <= 32)
+    sample_kernel<T, 32><<<a.B, kThreads, 0, st>>>(a);
+  else
+    sample_kernel<T, 50><<<a.B, kThreads, 0, st>>>(a);
+  NML_LAUNCHED();
+  return 0;
+}
+
 }  // namespace
 
 int launch_sample(int dt, const SampleArgs& a, hipStream_t st) {
@@ -1002,12 +1026,7 @@ int launch_sample(int dt, const SampleArgs& a, hipStream_t st) {
               "sample: generation mode needs the token history and prompt lengths");
   NML_REQUIRE(a.rep_penalty == 1.0f || a.V <= kBitmapWords * 32,
               "sample: repetition penalty supports vocab ≤ %d", kBitmapWords * 32);
-  if (dt == F16)
-    sample_kernel<half_t><<<a.B, kThreads, 0, st>>>(a);
-  else
-    sample_kernel<float><<<a.B, kThreads, 0, st>>>(a);
-  NML_LAUNCHED();
-  return 0;
+  return dt == F16 ? sample_launch<half_t>(a, st) : sample_launch<float>(a, st);
 }
 
 }  // namespace nml

@@ -31,7 +31,7 @@ def check(lg, top_k, top_p, u, temperature=0.8):
 
 
 @pytest.mark.parametrize("dtype", [np.float16, np.float32])
-@pytest.mark.parametrize("vocab", [5, 1023, 1025, 32768, 32769, 50304, 51201])
+@pytest.mark.parametrize("vocab", [5, 1023, 1025, 4096, 4097, 16384, 16385, 32768, 32769, 50304, 51200, 51201])
 @pytest.mark.parametrize("top_k,top_p", [(0, 0.9), (40, 0.95), (0, 0.05)])
 def test_vocab_edges(vocab, top_k, top_p, dtype):
     r = np.random.RandomState(vocab + top_k)
