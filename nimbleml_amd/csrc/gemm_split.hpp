@@ -13,8 +13,8 @@
 // roundings (relative error against 64 bits on unit-normal operands, the float32 MFMA's
 // in brackets: K 64 7.4e-8 (1.4e-7), K 1024 2.4e-7 (5.7e-7), K 32000 2.8e-7 (3.2e-6)).
 // An infinity, or a value that rounds up to one in bf16, makes an output NaN or infinite
-// that float32 arithmetic may not; so every non-finite output is formed again by float32
-// multiply-adds over its k range (dot_f32).
+// that float32 arithmetic may not; so every non-finite output is taken from the float32 MFMA
+// over its k range instead (tile_f32).
 //
 // Why: the float32 MFMA peaks at 157 TFLOP/s, the bf16 one at 2.5 PFLOP/s, a sixth of which
 // is 417. Measured, 4096 rows: 1024 × 1024 51 µs (167 TFLOP/s), 4096 × 1024 207 µs (166), the
@@ -67,26 +67,16 @@ __device__ __forceinline__ uint32_t cvt_pk(float x0, float x1) {
   return h;
 }
 
-// Σ_k A(m, k)·B(n, k) over [kbeg, kend) in float32, the slow path of a non-finite output.
-template <bool A_KC, bool B_KC>
-__device__ __forceinline__ float dot_f32(Operand a, Operand b, int m, int n, int kbeg, int kend) {
-  const float* pa = a.p + (A_KC ? m * a.ld : m);
-  const float* pb = b.p + (B_KC ? n * b.ld : n);
-  float s = 0.f;
-  for (int k = kbeg; k < kend; ++k)
-    s = __builtin_fmaf(pa[A_KC ? k : k * a.ld], pb[B_KC ? k : k * b.ld], s);
-  return s;
-}
-
 template <int TM, int TN, int WM, int WN, int WK>
 struct Shape {
   static constexpr int Threads = 64 * WM * WN * WK;
   static constexpr int MI = TM / WM / 32, NJ = TN / WN / 32;
   static constexpr int Plane = (TM + TN) * 64;  // A's rows, then B's
   static constexpr int Stage = 3 * Plane;
-  static constexpr size_t Lds = 2 * static_cast<size_t>(Stage);
+  static constexpr size_t Flag = 2 * static_cast<size_t>(Stage);  // one int: a non-finite output
+  static constexpr size_t Lds = Flag + 16;
   static_assert(MI >= 1 && NJ >= 1 && WK == 2, "tile");
-  static_assert(WK == 1 || static_cast<size_t>(TM) * TN * 4 <= Lds, "the WK sum goes through LDS");
+  static_assert(static_cast<size_t>(TM) * (TN + 1) * 4 <= Flag, "the WK sum and tile_f32's go through LDS");
 };
 
 // The values of one operand of R rows that this thread stages. KC: 4 k of a row per task, 8
@@ -190,6 +180,67 @@ struct Stager {
   }
 };
 
+// The tile's products on the float32 MFMA, k two at a time, left in lds as [row][TN + 1]: the
+// slow path of a tile with a non-finite output. Stages of 32 k in rows of 33 floats, the next
+// one's values in registers meanwhile; each wave takes G 32 × 32 blocks. A product of
+// non-finite outputs takes 2.7 times a finite one (4096 × 1024 × 1024: 142 µs against 53; with a
+// lane forming each of its outputs by itself 7.6 ms), one non-finite row 2.4 times.
+template <int TM, int TN, int T, bool A_KC, bool B_KC>
+__device__ __forceinline__ void tile_f32(Operand a, Operand b, int M, int N, int m0, int n0, int kbeg, int kend,
+                                         float* lds) {
+  constexpr int BN = TN / 32, G = TM / 32 * BN / (T / 64), P = kK + 1;
+  constexpr int RA = TM * kK / T, RB = TN * kK / T;  // values per thread and stage
+  static_assert(G >= 1 && BN % G == 0, "a wave's blocks lie in one row of blocks");
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int first = __builtin_amdgcn_readfirstlane(tid >> 6) * G, bm = first / BN * 32, bn = first % BN * 32;
+  floatx16 acc[G];
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[g][r] = 0.f;
+  float va[RA], vb[RB];
+  // value i of this thread: tile row and k, neighbouring lanes along the contiguous extent
+  auto row_of = [&](bool kc, int R, int i) { return kc ? (tid + T * i) / kK : (tid + T * i) % R; };
+  auto k_of = [&](bool kc, int R, int i) { return kc ? (tid + T * i) % kK : (tid + T * i) / R; };
+  auto fetch = [&](int k0) {
+#pragma unroll
+    for (int i = 0; i < RA; ++i) {
+      const int m = m0 + row_of(A_KC, TM, i), k = k0 + k_of(A_KC, TM, i);
+      va[i] = m < M && k < kend ? a.p[A_KC ? m * a.ld + k : k * a.ld + m] : 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < RB; ++i) {
+      const int n = n0 + row_of(B_KC, TN, i), k = k0 + k_of(B_KC, TN, i);
+      vb[i] = n < N && k < kend ? b.p[B_KC ? n * b.ld + k : k * b.ld + n] : 0.f;
+    }
+  };
+  fetch(kbeg);
+  for (int k0 = kbeg; k0 < kend; k0 += kK) {
+    __syncthreads();  // every wave is done with the stage before
+#pragma unroll
+    for (int i = 0; i < RA; ++i) lds[row_of(A_KC, TM, i) * P + k_of(A_KC, TM, i)] = va[i];
+#pragma unroll
+    for (int i = 0; i < RB; ++i) lds[(TM + row_of(B_KC, TN, i)) * P + k_of(B_KC, TN, i)] = vb[i];
+    __syncthreads();
+    if (k0 + kK < kend) fetch(k0 + kK);
+#pragma unroll 4
+    for (int kk = 0; kk < kK; kk += 2) {
+      const int k = kk + (lane >> 5);
+      const float x = lds[(bm + (lane & 31)) * P + k];
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+        acc[g] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, lds[(TM + bn + 32 * g + (lane & 31)) * P + k], acc[g], 0, 0, 0);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      lds[(bm + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * (TN + 1) + bn + 32 * g + (lane & 31)] = acc[g][r];
+  __syncthreads();
+}
+
 // One workgroup's tile at (m0, n0) over k in [kbeg, kend); epi(m, n, value) is called for
 // every element below M, N. lds: Shape::Lds bytes.
 template <int TM, int TN, int WM, int WN, int WK, bool A_KC, bool B_KC, typename Epi>
@@ -212,6 +263,8 @@ __device__ __forceinline__ void tile(Operand a, Operand b, int M, int N, int m0,
   typedef Stager<B_KC, TN, T, false> SB;
   SA sa(a, m0, M);
   SB sb(b, n0, N);
+  int* flag = reinterpret_cast<int*>(lds + Sh::Flag);
+  if (tid == 0) *flag = 0;
   constexpr int kSlices = SA::Slices + SB::Slices, kMfma = 6 * MI * NJ;
   // Multiplies the stage in buffer P (k step wk) and, with NEXT, splits parity P ^ 1's values
   // into the other buffer, a few instructions of the split behind each MFMA: the vector
@@ -359,7 +412,9 @@ __device__ __forceinline__ void tile(Operand a, Operand b, int M, int N, int m0,
   const int mb = m0 + wm * (TM / WM) + 4 * (lane >> 5), nb = n0 + wn * (TN / WN) + (lane & 31);
   constexpr int RN = 16 / WK;  // registers of a tile this wave finishes, from r0
   const int r0 = WK == 2 ? wk * 8 : 0;
-  uint64_t redo = 0;           // its non-finite outputs, one bit each
+  // This wave's outputs, and whether any is not finite: z stays 0 (a row past the last is a copy
+  // of the last).
+  float out[MI * NJ * RN], z = 0.f;
 #pragma unroll
   for (int i = 0; i < MI; ++i)
 #pragma unroll
@@ -368,20 +423,27 @@ __device__ __forceinline__ void tile(Operand a, Operand b, int M, int N, int m0,
       for (int r = 0; r < RN; ++r) {
         float v = acc[i][j][r];
         if constexpr (WK == 2) v = wk ? acc[i][j][8 + r] : v;
-        const int m = mb + 32 * i + 8 * ((r0 + r) >> 2) + (r & 3), n = nb + 32 * j;
-        if (m >= M || n >= N) continue;
-        if (__builtin_isfinite(v))
-          epi(m, n, v);
-        else
-          redo |= 1ull << ((i * NJ + j) * RN + r);
+        out[(i * NJ + j) * RN + r] = v;
+        z = __builtin_fmaf(v, 0.f, z);
       }
-  static_assert(MI * NJ * RN <= 64, "one bit per output");
-  while (redo) {
-    const int bit = __builtin_ctzll(redo);
-    redo &= redo - 1;
-    const int t = bit / RN, r = r0 + bit % RN;
+  // (asked before the stores, which the barrier would wait for)
+  if (z != 0.f) *flag = 1;
+  __syncthreads();
+  if (*flag) {
+    float* f32 = reinterpret_cast<float*>(lds);
+    tile_f32<TM, TN, T, A_KC, B_KC>(a, b, M, N, m0, n0, kbeg, kend, f32);
+#pragma unroll
+    for (int e = 0; e < MI * NJ * RN; ++e) {
+      const int t = e / RN, r = r0 + e % RN;
+      const int m = mb + 32 * (t / NJ) + 8 * (r >> 2) + (r & 3) - m0, n = nb + 32 * (t % NJ) - n0;
+      if (!__builtin_isfinite(out[e])) out[e] = f32[m * (TN + 1) + n];
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < MI * NJ * RN; ++e) {
+    const int t = e / RN, r = r0 + e % RN;
     const int m = mb + 32 * (t / NJ) + 8 * (r >> 2) + (r & 3), n = nb + 32 * (t % NJ);
-    epi(m, n, dot_f32<A_KC, B_KC>(a, b, m, n, kbeg, kend));
+    if (m < M && n < N) epi(m, n, out[e]);
   }
 }
 

@@ -76,6 +76,38 @@ def test_infinite_nan_and_largest_values(rows, n):
     assert (np.abs(got[plain] - want[plain]) <= bound(x[plain], w, k)).all()
 
 
+@pytest.mark.parametrize("rows,n", [(640, 1100), (1665, 1793)])
+def test_product_of_non_finite_rows(rows, n):
+    """Every output NaN or infinite, as in a diverged step: right, and taken by the float32 matrix
+    cores tile by tile (a few times a finite product's time; one lane per output takes over
+    fifteen times as long, on one row as on all)."""
+    r = np.random.RandomState(11)
+    k = 2052
+    x, w = r.randn(rows, k).astype(np.float32), r.randn(n, k).astype(np.float32)
+    bad = x.copy()
+    bad[:, k - 1] = np.where(np.arange(rows) % 2, np.inf, np.nan)
+    d = {name: N.DeviceArray.from_host(v) for name, v in (("w", w), ("x", x), ("bad", bad))}
+    out = N.DeviceArray((rows, n), np.float32)
+    timer = N.Timer()
+
+    def ms(name):
+        best = np.inf
+        for _ in range(5):
+            timer.start()
+            N.check(N.lib.nml_linear_device(d[name].ptr, k, d["w"].ptr, None, None, out.ptr, rows, k, n,
+                                            K.EPI_NONE, N.F32))
+            best = min(best, timer.stop())
+        return best
+
+    finite, got_finite = ms("x"), out.numpy()
+    slow, got = ms("bad"), out.numpy()
+    assert (np.abs(got_finite - x.astype(np.float64) @ w.T) <= bound(x, w.T, k)).all()
+    assert np.isnan(got[::2]).all()
+    assert (got[1::2] == np.sign(w[:, k - 1]) * np.float32(np.inf)).all()
+    print(f"finite {finite:.3f} ms, non-finite {slow:.3f} ms")
+    assert slow <= 8 * finite
+
+
 def test_sums_have_no_common_bias():
     """A column sum over many rows must not gather one-sided rounding: each output's error
     is independent, so the mean over 4096 rows falls like 1/sqrt(4096). Four standard errors
