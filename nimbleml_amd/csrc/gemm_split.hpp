@@ -4,7 +4,10 @@
 //
 // Each operand value is split as x = x0 + x1 + x2 with x0 = bf16(x), x1 = bf16(x − x0),
 // x2 = bf16(x − x0 − x1), all rounded to nearest: 8 + 8 + 8 significand bits and the signs
-// hold the 24 bits of x exactly. Of the nine products the six
+// hold the 24 bits of x exactly. (x is multiplied by 2^40 first and the sums by 2^-80 at the end,
+// so that this holds down to float32's smallest values: as they are, parts of a value below
+// 2^-109 leave bf16's range, at 2^-120 an output's error was 3.5e-5. A value from 2^88 on or an
+// output from 2^48 on then overflows, see below. It costs 0.8 % of a product.) Of the nine products the six
 //   x0·y0 + x0·y1 + x1·y0 + x0·y2 + x2·y0 + x1·y1
 // are summed in float32 on v_mfma_f32_32x32x16_bf16; the dropped ones (x1·y2, x2·y1,
 // x2·y2) are below 2^-25 of |x·y|, under the rounding of a single float32 product. A
@@ -43,6 +46,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kK = 32;      // k per stage
 constexpr int kChunk = 16;  // stages summed in one accumulator
+constexpr float kLift = 0x1p40f;
 // 128 × 128 tiles (one workgroup per CU) from this many of them on, 64 × 64 tiles (three
 // per CU) below: N = K = 1024, 128 of the large tiles 43.2 µs against 34.9 with the small, 192
 // 46.8 against 47.4, 256 51.4 against 62.9.
@@ -82,7 +86,8 @@ struct Shape {
 // The values of one operand of R rows that this thread stages. KC: 4 k of a row per task, 8
 // lanes a row (whole 128-byte lines per load); else 8 k of a row, 64 lanes taking 64
 // neighbouring rows at each k (256 contiguous bytes per load). NEG: the stage's second 16 k
-// are stored negated. Two stages' values are held, by the stage's parity.
+// are stored negated. All are stored times kLift. Two stages' values are held, by the stage's
+// parity.
 template <bool KC, int R, int T, bool NEG>
 struct Stager {
   static constexpr int V = KC ? 4 : 8;
@@ -95,7 +100,7 @@ struct Stager {
   uint32_t off[Tasks];      // this task's element past it (rows past the last: the last row,
                             // whose outputs nobody stores)
   uint32_t dst;             // task 0's bytes in a plane; task i's are Step·i further
-  uint32_t flip;            // sign bit to flip (every task's k are the same)
+  float lift;               // ±kLift (every task's k are the same)
   static constexpr int Step = KC ? T / 8 * 64 : 0;
   static_assert(KC ? (T / 8) % 16 == 0 : Tasks == 1, "tasks differ by whole swizzle periods");
 
@@ -117,7 +122,7 @@ struct Stager {
     }
     const uint32_t k = k_of(0);
     dst = plane_off(row_of(0), k / 8) + (KC ? (k & 4) * 2 : 0);
-    flip = (k & 16) << 27;
+    lift = k & 16 ? -kLift : kLift;
   }
 
   // a whole stage from k0
@@ -158,9 +163,9 @@ struct Stager {
     const int i = n / 3 / (V / 2), e = n / 3 % (V / 2), p = n % 3;
     float& v0 = v[P][i][2 * e];
     float& v1 = v[P][i][2 * e + 1];
-    if (NEG && p == 0) {
-      v0 = __uint_as_float(__float_as_uint(v0) ^ flip);
-      v1 = __uint_as_float(__float_as_uint(v1) ^ flip);
+    if (p == 0) {
+      v0 *= NEG ? lift : kLift;
+      v1 *= NEG ? lift : kLift;
     }
     const uint32_t h = cvt_pk(v0, v1);
     part[p][e] = h;
@@ -423,6 +428,7 @@ __device__ __forceinline__ void tile(Operand a, Operand b, int M, int N, int m0,
       for (int r = 0; r < RN; ++r) {
         float v = acc[i][j][r];
         if constexpr (WK == 2) v = wk ? acc[i][j][8 + r] : v;
+        v *= 1.f / kLift / kLift;
         out[(i * NJ + j) * RN + r] = v;
         z = __builtin_fmaf(v, 0.f, z);
       }

@@ -76,6 +76,31 @@ def test_infinite_nan_and_largest_values(rows, n):
     assert (np.abs(got[plain] - want[plain]) <= bound(x[plain], w, k)).all()
 
 
+# 64 and 128 wide tiles; operands near float32's smallest normal and largest values, where an
+# output also rounds to a multiple of the smallest value (2^-149)
+@pytest.mark.parametrize("rows,n", [(320, 832), (1665, 1793)])
+@pytest.mark.parametrize("ex,ew", [(-112, 0), (0, -112), (-126, 3), (4, -126), (-60, -62), (90, -60),
+                                   (-100, 92)])
+def test_operands_of_any_size(rows, n, ex, ew):
+    r = np.random.RandomState(n - ex + ew)
+    k = 68
+    x = (r.randn(rows, k) * 2.0**ex).astype(np.float32)
+    w = (r.randn(k, n) * 2.0**ew).astype(np.float32)
+    got = K.linear(x, w).numpy()
+    # (the large operands' outputs come from the float32 MFMA: k sums of two terms each)
+    terms = bound(x, w, k if max(ex, ew) < 80 else 16 * (k / 2 - 4) + 16)
+    assert (np.abs(got - x.astype(np.float64) @ w.astype(np.float64)) <= terms + 2.0**-149).all()
+    if ex > -80:
+        return
+    n_out = n // 4 * 4
+    dy = (r.randn(rows, n_out) * 2.0**ex).astype(np.float32)
+    xb, wb = r.randn(rows, k).astype(np.float32), r.randn(k, n_out).astype(np.float32)
+    dx, dw = backward(dy, xb, wb)
+    d64 = dy.astype(np.float64)
+    assert (np.abs(dx - d64 @ wb.T) <= bound(dy, wb.T, n_out) + 2.0**-149).all()
+    assert (np.abs(dw - xb.T.astype(np.float64) @ d64) <= bound(xb.T, dy, rows) + 2.0**-149).all()
+
+
 @pytest.mark.parametrize("rows,n", [(640, 1100), (1665, 1793)])
 def test_product_of_non_finite_rows(rows, n):
     """Every output NaN or infinite, as in a diverged step: right, and taken by the float32 matrix
