@@ -8,9 +8,12 @@
 //    (v_mfma_f32_32x32x16_f16, K=64 per LDS stage). Next stage prefetched into registers
 //    while the current one is multiplied.
 //  * gemm_f32: every float32 value split into three bf16 parts (gemm_split.hpp).
-//  * gemv: one activation row (decode), or up to 8 short ones. One wave per output row (or four), 16-byte loads
-//    along K, fp32 accumulation, wave-reduced.
-//  * rows: 2 … 8 rows (float32: up to 64), MFMA 16×16 tiles, K split over a workgroup's waves.
+//  * gemv: one activation row (decode), up to 8 float32 rows, up to 8 fp16 rows of at most 256
+//    values. One wave per output row (or four), 16-byte loads along K, fp32 accumulation,
+//    wave-reduced.
+//  * rows: a few rows, MFMA 16×16 tiles, K split over a workgroup's waves: fp16 2 … 8 rows, and
+//    9 … 64 whose K is above 256 and no multiple of 128; float32 9 … 16 rows, and any number
+//    while the output is at most 1024 tiles of 16×16.
 //  * skinny_f16: 8 < M ≤ 64 rows (batched decode), MFMA 16×16×32 with optional split-K
 //    and a fused RMSNorm of x (see its comment).
 #include <cstdlib>

@@ -163,9 +163,9 @@ __device__ __forceinline__ void tile_store(float (*S)[kGM + kGPad], const floatx
 
 // Split K (gridDim.z > 1): block z multiplies k in [z·kchunk, (z + 1)·kchunk) and writes
 // its partial product to c + z·zstride (OUT = GB_SET), summed afterwards in a fixed order.
-// T: operand type (and the output type of GB_SET / GB_GELU); GB_ADD adds fp32(T(acc)) to
-// an fp32 output (the reference forms the gradient in T, then accumulates it in fp32).
-template <bool A_KC, bool B_KC, int OUT, typename T>
+// fp16 operands (and output of GB_SET / GB_GELU); GB_ADD adds fp32(fp16(acc)) to an fp32
+// output (the reference forms the gradient in fp16, then accumulates it in fp32).
+template <bool A_KC, bool B_KC, int OUT>
 __global__ __launch_bounds__(256) void gemm_bwd_kernel(GemmBwdArgs g, int kchunk, long long zstride) {
   __shared__ __attribute__((aligned(16))) float As[kGK][kGM + kGPad];
   __shared__ __attribute__((aligned(16))) float Bs[kGK][kGM + kGPad];
@@ -175,8 +175,8 @@ __global__ __launch_bounds__(256) void gemm_bwd_kernel(GemmBwdArgs g, int kchunk
   const int M = g.M, N = g.N;
   const int kbeg = blockIdx.z * kchunk;
   const int K = min(g.K, kbeg + kchunk);
-  const T* __restrict__ ga = static_cast<const T*>(g.a);
-  const T* __restrict__ gbp = static_cast<const T*>(g.b);
+  const half_t* __restrict__ ga = static_cast<const half_t*>(g.a);
+  const half_t* __restrict__ gbp = static_cast<const half_t*>(g.b);
 
   floatx16 acc[2][2];
 #pragma unroll
@@ -234,15 +234,12 @@ __global__ __launch_bounds__(256) void gemm_bwd_kernel(GemmBwdArgs g, int kchunk
           if constexpr (OUT == kGBPart) {
             static_cast<float*>(g.c)[ci] = v;
           } else if constexpr (OUT == GB_ADD) {
-            static_cast<float*>(g.c)[ci] += rnd<T>(v);
+            static_cast<float*>(g.c)[ci] += rnd<half_t>(v);
           } else if constexpr (OUT == GB_SET) {
-            static_cast<T*>(g.c)[ci] = static_cast<T>(v);
+            static_cast<half_t*>(g.c)[ci] = static_cast<half_t>(v);
           } else {
-            const float x = static_cast<float>(static_cast<const T*>(g.aux)[static_cast<long long>(m) * g.ldaux + n]);
-            if constexpr (sizeof(T) == 4)
-              static_cast<T*>(g.c)[ci] = v * gelu_grad(x);
-            else
-              static_cast<T*>(g.c)[ci] = static_cast<T>(gelu_grad_f16(rnd<T>(v), x));
+            const float x = static_cast<float>(static_cast<const half_t*>(g.aux)[static_cast<long long>(m) * g.ldaux + n]);
+            static_cast<half_t*>(g.c)[ci] = static_cast<half_t>(gelu_grad_f16(rnd<half_t>(v), x));
           }
         }
       }
@@ -714,8 +711,8 @@ int gemm_bwd_f32(const GemmBwdArgs& g, int out, hipStream_t st) {
   return 0;
 }
 
-template <bool A_KC, bool B_KC, typename T>
-int gemm_bwd_out(const GemmBwdArgs& g, int out, hipStream_t st, bool mfma16 = false) {
+template <bool A_KC, bool B_KC>
+int gemm_bwd_out(const GemmBwdArgs& g, int out, hipStream_t st, bool mfma16) {
   const int tn = (g.N + kGM - 1) / kGM, tm = (g.M + kGM - 1) / kGM;
   // Few output tiles and a long K (a weight gradient, K = rows): split K so that the
   // grid holds ≥ 1024 blocks, each K slice ≥ 512 long.
@@ -737,38 +734,32 @@ int gemm_bwd_out(const GemmBwdArgs& g, int out, hipStream_t st, bool mfma16 = fa
     p.c = g_split.p;
     p.ldc = g.N;
     const dim3 grid(tn, tm, splits);
-    if constexpr (sizeof(T) == 2) {
-      if (mfma16)
-        gemm_bwd_f16_kernel<A_KC, B_KC, kGBPart><<<grid, 256, 0, st>>>(p, kchunk, static_cast<long long>(g.M) * g.N);
-      else
-        gemm_bwd_kernel<A_KC, B_KC, kGBPart, T><<<grid, 256, 0, st>>>(p, kchunk, static_cast<long long>(g.M) * g.N);
-    } else {
-      gemm_bwd_kernel<A_KC, B_KC, kGBPart, T><<<grid, 256, 0, st>>>(p, kchunk, static_cast<long long>(g.M) * g.N);
-    }
+    if (mfma16)
+      gemm_bwd_f16_kernel<A_KC, B_KC, kGBPart><<<grid, 256, 0, st>>>(p, kchunk, static_cast<long long>(g.M) * g.N);
+    else
+      gemm_bwd_kernel<A_KC, B_KC, kGBPart><<<grid, 256, 0, st>>>(p, kchunk, static_cast<long long>(g.M) * g.N);
     NML_LAUNCHED();
     const long long mn = static_cast<long long>(g.M) * g.N;
-    splitk_reduce_kernel<T><<<static_cast<int>((mn + 255) / 256), 256, 0, st>>>(
+    splitk_reduce_kernel<half_t><<<static_cast<int>((mn + 255) / 256), 256, 0, st>>>(
         g_split.p, splits, g.M, g.N, static_cast<float*>(g.c), g.ldc);
     NML_LAUNCHED();
     return 0;
   }
   const dim3 grid(tn, tm);
-  if constexpr (sizeof(T) == 2) {
-    if (mfma16) {
-      switch (out) {
-        case GB_SET: gemm_bwd_f16_kernel<A_KC, B_KC, GB_SET><<<grid, 256, 0, st>>>(g, g.K, 0); break;
-        case GB_ADD: gemm_bwd_f16_kernel<A_KC, B_KC, GB_ADD><<<grid, 256, 0, st>>>(g, g.K, 0); break;
-        case GB_GELU: gemm_bwd_f16_kernel<A_KC, B_KC, GB_GELU><<<grid, 256, 0, st>>>(g, g.K, 0); break;
-        default: set_error("gemm_bwd: unknown output mode %d", out); return -1;
-      }
-      NML_LAUNCHED();
-      return 0;
+  if (mfma16) {
+    switch (out) {
+      case GB_SET: gemm_bwd_f16_kernel<A_KC, B_KC, GB_SET><<<grid, 256, 0, st>>>(g, g.K, 0); break;
+      case GB_ADD: gemm_bwd_f16_kernel<A_KC, B_KC, GB_ADD><<<grid, 256, 0, st>>>(g, g.K, 0); break;
+      case GB_GELU: gemm_bwd_f16_kernel<A_KC, B_KC, GB_GELU><<<grid, 256, 0, st>>>(g, g.K, 0); break;
+      default: set_error("gemm_bwd: unknown output mode %d", out); return -1;
     }
+    NML_LAUNCHED();
+    return 0;
   }
   switch (out) {
-    case GB_SET: gemm_bwd_kernel<A_KC, B_KC, GB_SET, T><<<grid, 256, 0, st>>>(g, g.K, 0); break;
-    case GB_ADD: gemm_bwd_kernel<A_KC, B_KC, GB_ADD, T><<<grid, 256, 0, st>>>(g, g.K, 0); break;
-    case GB_GELU: gemm_bwd_kernel<A_KC, B_KC, GB_GELU, T><<<grid, 256, 0, st>>>(g, g.K, 0); break;
+    case GB_SET: gemm_bwd_kernel<A_KC, B_KC, GB_SET><<<grid, 256, 0, st>>>(g, g.K, 0); break;
+    case GB_ADD: gemm_bwd_kernel<A_KC, B_KC, GB_ADD><<<grid, 256, 0, st>>>(g, g.K, 0); break;
+    case GB_GELU: gemm_bwd_kernel<A_KC, B_KC, GB_GELU><<<grid, 256, 0, st>>>(g, g.K, 0); break;
     default: set_error("gemm_bwd: unknown output mode %d", out); return -1;
   }
   NML_LAUNCHED();
@@ -2273,8 +2264,8 @@ int launch_gemm_bwd(int dt, const GemmBwdArgs& g, bool a_kc, bool b_kc, int out,
     const char* bigenv = std::getenv("NIMBLEML_TRAIN_F16_BIG");
     if (m16 && g.K % big::kK == 0 && !(bigenv && bigenv[0] == '0')) return gemm_bwd_big(g, a_kc, b_kc, out, st);
     if (a_kc)
-      return b_kc ? gemm_bwd_out<true, true, half_t>(g, out, st, m16) : gemm_bwd_out<true, false, half_t>(g, out, st, m16);
-    return b_kc ? gemm_bwd_out<false, true, half_t>(g, out, st, m16) : gemm_bwd_out<false, false, half_t>(g, out, st, m16);
+      return b_kc ? gemm_bwd_out<true, true>(g, out, st, m16) : gemm_bwd_out<true, false>(g, out, st, m16);
+    return b_kc ? gemm_bwd_out<false, true>(g, out, st, m16) : gemm_bwd_out<false, false>(g, out, st, m16);
   }
   if (a_kc) return b_kc ? gemm_bwd_f32<true, true>(g, out, st) : gemm_bwd_f32<true, false>(g, out, st);
   return b_kc ? gemm_bwd_f32<false, true>(g, out, st) : gemm_bwd_f32<false, false>(g, out, st);
