@@ -1455,9 +1455,12 @@ struct TileRegs {
   }
 };
 
-// dK, dV of 64 keys; the query tiles from the key tile on.
+// dK, dV of 64 keys; the query tiles from the key tile on. (Head dims above 64: the LDS holds one
+// workgroup per CU whatever its registers, and with the bound for two 100 to 260 of them were
+// spilled: 64 (sequence, head) pairs × 1024 positions in float32, the whole backward 1854 → 1622
+// µs at 96, 2759 → 1944 at 128.)
 template <int DK, bool PAD, typename T>
-__global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_mfma(AttnBwdArgs a) {
+__global__ __launch_bounds__(256, DK > 64 ? 1 : 2) void attn_bwd_dkdv_mfma(AttnBwdArgs a) {
   extern __shared__ float lds[];
   constexpr int P = DK + 1, NJ = DK / 32;
   const int hd = PAD ? a.dk : DK;
