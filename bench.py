@@ -246,7 +246,8 @@ def bench_adamw(nm, n=337_100_000, steps=20):
                          "bytes_per_element": 28}}
 
 
-MFMA_F32_PEAK_TFLOPS = 157.3
+# A float32 model's products run as six bf16 MFMA products each, of 2.5 PFLOP/s dense.
+MFMA_F32_SPLIT_PEAK_TFLOPS = 416.7
 
 
 def bench_train(nm, batch=4, seq=1024, steps=3, dtype=np.float32, skew=False):
@@ -294,9 +295,9 @@ def bench_train(nm, batch=4, seq=1024, steps=3, dtype=np.float32, skew=False):
     fwd = 2 * R * L * 12 * d * d + L * batch * 4 * d * seq * (seq + 1) / 2 + 2 * R * d * V
     tf = 3 * fwd / (ms * 1e-3) / 1e12
     name = "float32" if dtype == np.float32 else "float16 (float32 gradients and masters)"
-    # the peak of the GEMMs' arithmetic: fp32 MFMA, or fp16 MFMA for a float16 model (whose
-    # attention backward still runs on the fp32 MFMA, from fp16 operands)
-    peak = MFMA_F32_PEAK_TFLOPS if dtype == np.float32 else MFMA_F16_PEAK_TFLOPS
+    # the peak of the GEMMs' arithmetic: bf16 MFMA in six products (a float32 model's attention runs
+    # on the fp32 MFMA, 157 TFLOP/s), or fp16 MFMA for a float16 model
+    peak = MFMA_F32_SPLIT_PEAK_TFLOPS if dtype == np.float32 else MFMA_F16_PEAK_TFLOPS
     return {"workload": f"train step: GPT V32000 d1024 H16 L24 {name}, batch {batch} x {seq}, "
                         "zero_grad + compute_loss + backward + AdamW on the device"
                         + (" (half of the ids one token)" if skew else ""),

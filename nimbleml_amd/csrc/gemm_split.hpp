@@ -22,10 +22,10 @@
 // Why: the float32 MFMA peaks at 157 TFLOP/s, the bf16 one at 2.5 PFLOP/s, a sixth of which
 // is 417. Measured, 4096 rows: 1024 × 1024 51 µs (167 TFLOP/s), 4096 × 1024 207 µs (166), the
 // 32000-row tied head 2202 → 1600 µs (122 → 168) against a float32 MFMA kernel of the same
-// tile. What bounds it: the matrix unit is busy 58 % of the cycles, at the 1.65 GHz that the
-// chip holds under this load; of the rest, without the split the same loop runs 1.3
-// times as fast, and the vector work (six instructions an MFMA) hides under the MFMAs only
-// in part.
+// tile. What bounds it: the matrix unit is busy 55 % of the cycles (the head, counters), at the
+// 1.5 to 1.8 GHz that the chip holds under this load; of the rest, without the split the same
+// loop runs 1.3 times as fast, and the vector work (6.8 instructions an MFMA) hides under the
+// MFMAs only in part. The 128 × 128 tile holds all 256 registers and spills 16 to 21.
 //
 // A workgroup of WM·WN·WK waves owns a TM × TN tile; a wave TM/WM × TN/WN of it and, of the
 // two 16-wide k steps of a stage, one (the two partial tiles are summed through LDS at
