@@ -4,10 +4,11 @@
 //
 // Each operand value is split as x = x0 + x1 + x2 with x0 = bf16(x), x1 = bf16(x − x0),
 // x2 = bf16(x − x0 − x1), all rounded to nearest: 8 + 8 + 8 significand bits and the signs
-// hold the 24 bits of x exactly. (x is multiplied by 2^40 first and the sums by 2^-80 at the end,
-// so that this holds down to float32's smallest values: as they are, parts of a value below
-// 2^-109 leave bf16's range, at 2^-120 an output's error was 3.5e-5. A value from 2^88 on or an
-// output from 2^48 on then overflows, see below. It costs 0.8 % of a product.) Of the nine products the six
+// hold the 24 bits of x exactly. (x is multiplied by kLift = 2^16 first and the sums by 2^-32 at the
+// end, so that this holds for every float32: the last bit of the smallest, 2^-149, becomes bf16's
+// smallest value. As they are, values below 2^-109 lose parts; at 2^-120 an output's error was
+// 3.5e-5. A value from 2^112 on or an output from 2^96 on then overflows, see below. It costs
+// 0.8 % of a product.) Of the nine products the six
 //   x0·y0 + x0·y1 + x1·y0 + x0·y2 + x2·y0 + x1·y1
 // are summed in float32 on v_mfma_f32_32x32x16_bf16; the dropped ones (x1·y2, x2·y1,
 // x2·y2) are below 2^-25 of |x·y|, under the rounding of a single float32 product. A
@@ -46,7 +47,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kK = 32;      // k per stage
 constexpr int kChunk = 16;  // stages summed in one accumulator
-constexpr float kLift = 0x1p40f;
+constexpr float kLift = 0x1p16f;
 // 128 × 128 tiles (one workgroup per CU) from this many of them on, 64 × 64 tiles (three
 // per CU) below: N = K = 1024, 128 of the large tiles 43.2 µs against 34.9 with the small, 192
 // 46.8 against 47.4, 256 51.4 against 62.9.

@@ -105,7 +105,7 @@ def test_infinite_nan_and_largest_values(tile, rows, n):
 # output also rounds to a multiple of the smallest value (2^-149)
 @pytest.mark.parametrize("rows,n", [(320, 832), (1665, 1793)])
 @pytest.mark.parametrize("ex,ew", [(-112, 0), (0, -112), (-126, 3), (4, -126), (-60, -62), (90, -60),
-                                   (-100, 92)])
+                                   (-100, 92), (116, -70), (-80, 115), (60, 45)])
 def test_operands_of_any_size(rows, n, ex, ew):
     assert split_tile(rows, n) == (64 if rows == 320 else 128)
     r = np.random.RandomState(n - ex + ew)
@@ -113,10 +113,12 @@ def test_operands_of_any_size(rows, n, ex, ew):
     x = (r.randn(rows, k) * 2.0**ex).astype(np.float32)
     w = (r.randn(k, n) * 2.0**ew).astype(np.float32)
     got = K.linear(x, w).numpy()
-    # (the large operands' outputs come from the float32 MFMA: k sums of two terms each)
-    terms = bound(x, w, k if max(ex, ew) < 80 else 16 * (k / 2 - 4) + 16)
+    # (outputs of the largest operands, and the largest outputs, come from the float32 MFMA: k / 2
+    # sums of two terms each)
+    f32 = max(ex, ew) > 100 or ex + ew > 90
+    terms = bound(x, w, 16 * (k / 2 - 4) + 16 if f32 else k)
     assert (np.abs(got - x.astype(np.float64) @ w.astype(np.float64)) <= terms + 2.0**-149).all()
-    if ex > -80:
+    if ex > -110:
         return
     n_out = n // 4 * 4
     dy = (r.randn(rows, n_out) * 2.0**ex).astype(np.float32)
