@@ -21,9 +21,9 @@
 // over its k range instead (tile_f32).
 //
 // Why: the float32 MFMA peaks at 157 TFLOP/s, the bf16 one at 2.5 PFLOP/s, a sixth of which
-// is 417. Measured, 4096 rows: 1024 × 1024 51 µs (167 TFLOP/s), 4096 × 1024 207 µs (166), the
-// 32000-row tied head 2202 → 1600 µs (122 → 168) against a float32 MFMA kernel of the same
-// tile. What bounds it: the matrix unit is busy 55 % of the cycles (the head, counters), at the
+// is 417. Measured, 4096 rows, a float32 MFMA kernel of the same tile and this one: N = K = 1024
+// 94 → 53 µs (162 TFLOP/s), N 4096 317 → 222 (155), K 4096 343 → 203 (169), the 32000-row tied
+// head's loss 2484 → 1636. What bounds it: the matrix unit is busy 55 % of the cycles (the head, counters), at the
 // 1.5 to 1.8 GHz that the chip holds under this load; of the rest, without the split the same
 // loop runs 1.3 times as fast, and the vector work (6.8 instructions an MFMA) hides under the
 // MFMAs only in part. The 128 × 128 tile holds all 256 registers and spills 16 to 21.
